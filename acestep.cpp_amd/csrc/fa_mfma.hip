@@ -59,10 +59,22 @@ constexpr int kPfEarlyMaxKt = 4;             // key tiles up to which a tile's c
 constexpr int kPfWindowEarlyMaxKt = 8;       // the same for the key tiles a structured window spans
 static_assert(kPfLook >= 1 && kPfLook <= 7, "operand ring holds 8");
 
+// Eight bytes at any 2-byte aligned address (one global_load_dwordx2: gfx950
+// loads need no more alignment than their element under ROCm).
+struct __attribute__((packed, aligned(2))) U64Any {
+    uint64_t v;
+};
+
+// UNAL: mask rows at any 2-byte alignment and of any length >= 4.  The DiT
+// and the encoders build [S, S] masks without padding (src/dit-sampler.h:
+// 262-309, src/qwen3-enc.h:429-437), so every S that is not a multiple of 4
+// gives such rows.  A 4-key group that would run past key Skv - 1 is read
+// from key Skv - 4 and shifted, so that no load leaves the row.
+template <bool UNAL>
 __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint8_t *cls) {
     // One workgroup per (key tile, query tile, mask plane).  Each row of the
-    // tile (64 keys = 128 B) is read by 16 lanes with 8-byte loads (the
-    // prefill path guarantees 8-byte aligned mask rows).  All 8 loads of a
+    // tile (64 keys = 128 B) is read by 16 lanes with 8-byte loads (8-byte
+    // aligned rows, or UNAL).  All 8 loads of a
     // lane are issued before any is looked at: addresses are clamped into
     // the live rows and keys, so no load needs a branch, and rows / keys
     // outside [0, Sq) x [0, Skv) are excluded afterwards by predicates.  The
@@ -96,13 +108,20 @@ __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint
     // a group starting at or past Skv is read at the last live group
     // instead (its values are excluded below); with the mask's ne0 % 4 == 0
     // (host-checked) every group read lies inside its row
-    const uint32_t kc = (uint32_t)min(k, (a.Skv - 1) & ~3);
+    const uint32_t kc = (uint32_t)min(k, UNAL ? a.Skv - 4 : (a.Skv - 1) & ~3);
     u16x4 v[kPfBM / 16];
 #pragma unroll
     for (int pass = 0; pass < kPfBM / 16; pass++) {
         const uint32_t q = (uint32_t)min(q_lo + r0 + 16 * pass, a.Sq - 1);
-        v[pass] = __builtin_bit_cast(u16x4, __builtin_amdgcn_raw_buffer_load_b64(
-                                                rs, q * (uint32_t)a.m_nb1 + 2u * kc, 0, 0));
+        const uint32_t off = q * (uint32_t)a.m_nb1 + 2u * kc;
+        if constexpr (UNAL) v[pass] = __builtin_bit_cast(u16x4, ((const U64Any *)(base + off))->v);
+        else v[pass] = __builtin_bit_cast(u16x4, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0));
+    }
+    if constexpr (UNAL) {   // (keys past Skv are excluded below, whatever the shift leaves there)
+        const int sh = 16 * min(k - (int)kc, 3);
+#pragma unroll
+        for (int pass = 0; pass < kPfBM / 16; pass++)
+            v[pass] = __builtin_bit_cast(u16x4, __builtin_bit_cast(uint64_t, v[pass]) >> sh);
     }
     bool all_ninf = true, all_zero = true, all_bin = true;
     uint32_t live = 0;   // bit 4 pass + i: key k + i of row q_lo + r0 + 16 pass is live (0 past Skv)
@@ -148,10 +167,13 @@ __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint
 // arithmetic on (query row, key) -- no classifier pass, no mask reads.
 // QQ8: Q quantised to Q8_0 on load, as ggml quantises Q for a Q8_0 K (the
 // K/V rows of a Q8_0 cache are staged in F16 by q8_stage.hip first).
+// UNAL: the dense mask's rows have no 8-byte alignment: values of mixed
+// tiles are read one by one (0 / -inf masks never get there: they come as
+// liveness words).
 // SPREAD: the next tile's copies go out one per QK MFMA of the current
 // tile (true), or all before the tile, with Q loaded as whole rows (false:
 // jobs of few key tiles, chosen in launch_fa_prefill).
-template <int T, bool CAP, bool SM, bool QQ8, bool SPREAD = true>
+template <int T, bool CAP, bool SM, bool QQ8, bool SPREAD, bool UNAL>
 __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     using MF = Mfma32<T>;
     using V8 = typename MF::v8;
@@ -469,9 +491,15 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         // (the four mask words go out together: one memory round trip)
         u16x4 mw4[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-            mw4[j] = __builtin_bit_cast(
-                u16x4, __builtin_amdgcn_raw_buffer_load_b64(mrs, mrow_off + 2u * (uint32_t)key0 + 16u * j, 0, 0));
+        for (int j = 0; j < 4; j++) {
+            const uint32_t off = mrow_off + 2u * (uint32_t)key0 + 16u * j;
+            if constexpr (UNAL) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) mw4[j][i] = __builtin_amdgcn_raw_buffer_load_b16(mrs, off + 2u * i, 0, 0);
+            } else {
+                mw4[j] = __builtin_bit_cast(u16x4, __builtin_amdgcn_raw_buffer_load_b64(mrs, off, 0, 0));
+            }
+        }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const u16x4 mw = mw4[j];
@@ -722,24 +750,37 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     }
 }
 
-template <int T, bool CAP, bool SM, bool SPREAD>
+template <int T, bool CAP, bool SM, bool SPREAD, bool UNAL>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 fa_prefill_kernel(const FaArgs a) {
-    fa_prefill_body<T, CAP, SM, false, SPREAD>(a);
+    fa_prefill_body<T, CAP, SM, false, SPREAD, UNAL>(a);
 }
 
 // Prefill over a Q8_0 cache: K/V rows staged in F16, Q quantised on load.
 template <bool CAP, bool SM>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 fa_prefill_q8q_kernel(const FaArgs a) {
-    fa_prefill_body<T_F16, CAP, SM, true>(a);
+    fa_prefill_body<T_F16, CAP, SM, true, true, false>(a);
 }
 
 hipError_t launch_mask_classify(const FaArgs &a, int n_planes, uint8_t *classes, hipStream_t stream) {
     // (1D over every tile of the n_planes = m_ne2 * m_ne3 mask planes)
     if (n_planes != a.m_ne2 * a.m_ne3) return hipErrorInvalidValue;
     dim3 grid((uint32_t)a.n_kt * (uint32_t)a.n_qt * (uint32_t)n_planes);
-    hipLaunchKernelGGL(mask_classify_kernel, grid, dim3(256), 0, stream, a, classes);
+    if (a.mask_unal) hipLaunchKernelGGL(mask_classify_kernel<true>, grid, dim3(256), 0, stream, a, classes);
+    else hipLaunchKernelGGL(mask_classify_kernel<false>, grid, dim3(256), 0, stream, a, classes);
+    return hipGetLastError();
+}
+
+template <int KT, bool CAP, bool SM, bool UNAL>
+static hipError_t launch_pf(const FaArgs &a, dim3 grid, bool spread, hipStream_t stream) {
+    if constexpr (KT == T_Q8_0) {
+        if constexpr (UNAL) return hipErrorInvalidValue;   // (the host keeps those on the decode kernel)
+        else hipLaunchKernelGGL((fa_prefill_q8q_kernel<CAP, SM>), grid, dim3(256), kPfLds, stream, a);
+    } else if (spread)
+        hipLaunchKernelGGL((fa_prefill_kernel<KT, CAP, SM, true, UNAL>), grid, dim3(256), kPfLds, stream, a);
+    else
+        hipLaunchKernelGGL((fa_prefill_kernel<KT, CAP, SM, false, UNAL>), grid, dim3(256), kPfLds, stream, a);
     return hipGetLastError();
 }
 
@@ -758,27 +799,22 @@ hipError_t launch_fa_prefill(const FaArgs &a, int ktype, hipStream_t stream) {
                                                       : 2 * (int64_t)a.sm_window + kPfBM;
         if ((span + kPfBN - 1) / kPfBN + 1 <= kPfWindowEarlyMaxKt) spread = false;
     }
-#define MXFA_PF(TT, C, S)                                                                                    \
-    do {                                                                                                     \
-        if (spread) hipLaunchKernelGGL((fa_prefill_kernel<TT, C, S, true>), grid, dim3(256), kPfLds, stream, a); \
-        else hipLaunchKernelGGL((fa_prefill_kernel<TT, C, S, false>), grid, dim3(256), kPfLds, stream, a);       \
-    } while (0)
-    if (ktype == T_F16) {
-        if (sm) { if (cap) MXFA_PF(T_F16, true, true); else MXFA_PF(T_F16, false, true); }
-        else { if (cap) MXFA_PF(T_F16, true, false); else MXFA_PF(T_F16, false, false); }
-    } else if (ktype == T_BF16) {
-        if (sm) { if (cap) MXFA_PF(T_BF16, true, true); else MXFA_PF(T_BF16, false, true); }
-        else { if (cap) MXFA_PF(T_BF16, true, false); else MXFA_PF(T_BF16, false, false); }
-    } else if (ktype == T_Q8_0) {
-#define MXFA_PFQ(C, S) hipLaunchKernelGGL((fa_prefill_q8q_kernel<C, S>), grid, dim3(256), kPfLds, stream, a)
-        if (sm) { if (cap) MXFA_PFQ(true, true); else MXFA_PFQ(false, true); }
-        else { if (cap) MXFA_PFQ(true, false); else MXFA_PFQ(false, false); }
-#undef MXFA_PFQ
-    } else {
-        return hipErrorInvalidValue;
+    const bool unal = a.mask_unal != 0;   // (never with a structured mask)
+    auto typed = [&](auto kt) {
+        constexpr int KT = decltype(kt)::value;
+        if (sm) return cap ? launch_pf<KT, true, true, false>(a, grid, spread, stream)
+                           : launch_pf<KT, false, true, false>(a, grid, spread, stream);
+        if (unal) return cap ? launch_pf<KT, true, false, true>(a, grid, spread, stream)
+                             : launch_pf<KT, false, false, true>(a, grid, spread, stream);
+        return cap ? launch_pf<KT, true, false, false>(a, grid, spread, stream)
+                   : launch_pf<KT, false, false, false>(a, grid, spread, stream);
+    };
+    switch (ktype) {
+        case T_F16: return typed(std::integral_constant<int, T_F16>{});
+        case T_BF16: return typed(std::integral_constant<int, T_BF16>{});
+        case T_Q8_0: return typed(std::integral_constant<int, T_Q8_0>{});
+        default: return hipErrorInvalidValue;
     }
-#undef MXFA_PF
-    return hipGetLastError();
 }
 
 }  // namespace mxfa

@@ -477,17 +477,28 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     a.mask_al16 = mask_rows_aligned(16);
     a.mask_vec4 = a.mask_al8 && mask->ne[0] >= ((k->ne[1] + 3) & ~(int64_t)3);
     a.mask_vec16 = a.mask_vec4 && mask->ne[0] >= 16;
-    // prefill: mask rows are read in 8-byte groups of 4 keys (rows 8-byte
-    // aligned) through a buffer resource over one mask plane, addressed
-    // with 32-bit offsets.  With ne0 % 4 == 0 every group that starts below
-    // Skv lies wholly inside its row, so no load that carries a live key
-    // crosses the end of the plane (a contiguous 8-byte aligned mask has
-    // ne0 % 4 == 0 anyway; other strided views go to the decode kernel).
+    // prefill: mask rows are read in groups of 4 keys, addressed with 32-bit
+    // offsets into one mask plane.  8-byte aligned rows of a multiple of 4
+    // entries (every LM mask: windows are padded to 256 keys) are read
+    // through a buffer resource, every group that starts below Skv lying
+    // inside its row.  Other rows, at any 2-byte alignment, take the
+    // instances that shift a row's last group into place (mask_unal): the
+    // DiT's and the encoders' [S, S] masks for 3 of 4 lengths S.  Measured
+    // per call against the scalar decode kernel, which streams all of K and
+    // V for every 16 query rows: 2 x 1085 tokens at 16 / 8 heads under a
+    // window of 128, 29.2 against 123.7 us; over 238 encoder keys, 22.3
+    // against 70.7 us; eight layers of 437 tokens, four of them under a
+    // window, 146.9 against 262.7 us.
     if (mask) {
         const uint64_t plane = (uint64_t)(mask->ne[1] - 1) * mask->nb[1] + 2 * (uint64_t)mask->ne[0];
         a.m_plane_bytes = plane <= 0x7FFFFFFFull ? (uint32_t)plane : 0;
+        a.mask_unal = !(a.mask_al8 && mask->ne[0] % 4 == 0);
     }
-    const bool mask_vec_ok = !mask || (a.mask_al8 && a.m_plane_bytes != 0 && mask->ne[0] % 4 == 0);
+    // (Q8_0 calls under such masks stay on the decode kernel, whose integer
+    // dots are closer to ggml's than the F16 staging below; the LM, which
+    // owns the quantised cache, always pads its masks)
+    const bool mask_vec_ok = !mask || (a.m_plane_bytes != 0 &&
+                                       (!a.mask_unal || (a.Skv >= 4 && k->type != MXFA_TYPE_Q8_0)));
     const int64_t n_kt = (a.Skv + kPfBN - 1) / kPfBN;
     // the prefill kernel addresses one (batch, kv head)'s K and V rows with
     // 32-bit offsets from a buffer base: every row of every key tile must
@@ -513,7 +524,8 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     // word path)
     const bool bits_fit = mask && !q8 && with_bits <= ws_cap;
     pl.prefill = (k->type == MXFA_TYPE_F16 || k->type == MXFA_TYPE_BF16 || q8) && a.Sq >= kPrefillMinSq &&
-                 mask_vec_ok && offsets_32 && stage_ok && stage_fits && (!mask || n_kt <= kPfMaxKeyTiles);
+                 mask_vec_ok && offsets_32 && stage_ok && stage_fits && (!mask || n_kt <= kPfMaxKeyTiles) &&
+                 (!a.mask_unal || cls_pf <= ws_cap);
     if (pl.prefill) {
         a.n_qt = (a.Sq + kPfBM - 1) / kPfBM;
         a.n_kt = (int32_t)n_kt;
@@ -528,7 +540,9 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         // wide kernel's registers without spills.)
         // The same rule holds for a dense mask and its structured form, so
         // that the two stay on one kernel (bit-identical outputs).
-        pl.wide = kPfWide && k->type == MXFA_TYPE_F16 && a.softcap == 0.0f &&
+        // (mask rows without 8-byte alignment: the 32-query kernel, which
+        // reads the words of 0 / -inf tiles instead of their values)
+        pl.wide = kPfWide && k->type == MXFA_TYPE_F16 && a.softcap == 0.0f && !a.mask_unal &&
                   ((!mask && a.sm_flags == 0) || n_kt <= kPfWideMaskedMaxKt);
         a.n_qt_w = pl.wide ? (a.Sq + kPfWideBM - 1) / kPfWideBM : 0;
         pl.n_planes = mask ? a.m_ne2 * a.m_ne3 : 0;
@@ -867,8 +881,17 @@ int run(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const 
         ws = fixed->ws;
         tickets = fixed->tickets;
     } else {
-        const int rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
+        int rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
+        if (rc != MXFA_OK && pl.prefill && pl.args.mask_unal) {
+            // (the workspace cannot grow, for instance under capture: such
+            // a mask needs none on the decode kernel)
+            pl = Plan{};
+            make_plan(q, k, v, mask, params, dst, pl, sm, 0);
+            rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
+        }
         if (rc != MXFA_OK) return rc;
+        if (!pl.prefill && (int64_t)pl.args.Nkv * pl.args.row_tiles > 65535)
+            return fail(MXFA_ERR_UNSUPPORTED, "too many query rows per KV head for the decode kernel");
     }
     FaArgs &a = pl.args;
     hipError_t e;
@@ -891,7 +914,9 @@ int run(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const 
             if (!fixed) {
                 uint8_t *gc = nullptr;
                 const int rc = graph_classes(mask, a.Sq, a.Skv, pl.cls_block, stream, &gc, &classify);
-                if (rc != MXFA_OK) return rc;
+                // (unaligned rows: a class arena that cannot grow leaves the
+                // call to classify into its own workspace)
+                if (rc != MXFA_OK && !a.mask_unal) return rc;
                 if (gc) cls = gc;
                 else classify = true;
             }

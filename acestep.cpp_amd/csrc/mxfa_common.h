@@ -63,6 +63,7 @@ struct FaArgs {
     // 8-byte aligned rows holding at least round_up(Skv, 4) entries;
     // mask_vec16: the same with at least 16 entries (16-key DMA blocks)
     int32_t mask_al8, mask_al16, mask_vec4, mask_vec16;
+    int32_t mask_unal;                    // prefill: rows not 8-byte aligned, or not of a multiple of 4 entries
     uint32_t m_plane_bytes;               // prefill: bytes of one mask plane, (ne1 - 1) * nb1 + 2 * ne0
     // split-KV
     int32_t n_splits, chunk;
