@@ -274,10 +274,9 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // +0, V rows at +16 KB, 256 B per key, 16-byte chunks XOR-swizzled).
     // Wave w copies keys 16w..16w+15 of the tile (four copies of 4 keys x
     // 16 chunks for K and for V): lane -> (key 16w + 4c + lane/16, slot
-    // lane%16), the slot holding the swizzled logical chunk.  Each copy goes
-    // through a buffer resource based at the wave's first row and sized to
-    // the rows that exist, so keys past Skv (the last partial tile, and the
-    // look-ahead past the last tile) read as zeros and touch no memory.
+    // lane%16), the slot holding the swizzled logical chunk.  Keys past Skv
+    // (the last partial tile) lie past the resource: they read as zeros and
+    // touch no memory.
     const int dkey = lane >> 4, dslot = lane & 15;
     uint32_t vk[4], vv[4];
 #pragma unroll
@@ -285,23 +284,24 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         vk[c] = (uint32_t)(4 * c + dkey) * k_row + 16u * (uint32_t)(dslot ^ swz_k(4 * c + dkey));
         vv[c] = (uint32_t)(4 * c + dkey) * v_row + 16u * (uint32_t)(dslot ^ swz_v(4 * c + dkey));
     }
-    // (32-bit row offsets: the host routes here only (batch, kv head)
-    // slices whose key tiles lie within 4 GiB of their base; a look-ahead
-    // tile at or past n_kt gets an empty resource and reads nothing)
-    auto tile_rsrc = [&](const char *base, uint64_t avail, uint32_t row, int kt) __attribute__((always_inline)) {
-        const uint32_t off = (uint32_t)(kt * kPfBN + 16 * wave) * row;
-        const uint64_t n = kt < a.n_kt && avail > off ? min(avail - off, (uint64_t)0xFFFFFFFFu) : 0;
-        return buf_rsrc(base + off, (uint32_t)n);
-    };
+    // One resource per kernel for K and one for V, from the (batch, kv
+    // head)'s first row, sized to the rows that exist: a copy's lane offset
+    // is its place in the tile plus the tile's first row.  (A resource per
+    // tile took ~20 scalar instructions and six readfirstlanes at each tile's
+    // top: 2 x 3000 tokens without a mask 152.4 -> 149.3 us on fa_wide.hip,
+    // 1000 tokens over a Q8_0 cache 53.7 -> 52.2 us here.)  (32-bit row
+    // offsets: the host routes here only (batch, kv head) slices whose key
+    // tiles lie within 4 GiB of their base.)
+    const i32x4 rk = buf_rsrc(kbase, (uint32_t)min(k_avail, (uint64_t)0xFFFFFFFFu));
+    const i32x4 rv = buf_rsrc(vbase, (uint32_t)min(v_avail, (uint64_t)0xFFFFFFFFu));
     auto issue = [&](int kt, auto st_c) __attribute__((always_inline)) {
         constexpr int ST = decltype(st_c)::value;
         const uint32_t l0 = lds0 + ST * kStageBytes + (uint32_t)(16 * wave) * 256u;
-        const i32x4 rk = tile_rsrc(kbase, k_avail, k_row, kt);
-        const i32x4 rv = tile_rsrc(vbase, v_avail, v_row, kt);
+        const uint32_t ko = (uint32_t)(kt * kPfBN + 16 * wave) * k_row, vo = (uint32_t)(kt * kPfBN + 16 * wave) * v_row;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            dma16_buf(rk, vk[c], l0 + 4 * c * 256);
-            dma16_buf(rv, vv[c], l0 + kTileBytes + 4 * c * 256);
+            dma16_buf(rk, vk[c] + ko, l0 + 4 * c * 256);
+            dma16_buf(rv, vv[c] + vo, l0 + kTileBytes + 4 * c * 256);
         }
     };
 
@@ -565,11 +565,11 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         constexpr int NST = decltype(nst_c)::value;
         const bool do_issue = SPREAD && kn < n_kt;   // uniform
         const uint32_t nl0 = lds0 + NST * kStageBytes + (uint32_t)(16 * wave) * 256u;
-        i32x4 nrk = {0, 0, 0, 0}, nrv = {0, 0, 0, 0};
-        if (do_issue) {
-            nrk = tile_rsrc(kbase, k_avail, k_row, kn);
-            nrv = tile_rsrc(vbase, v_avail, v_row, kn);
-        }
+        const uint32_t nko = (uint32_t)(kn * kPfBN + 16 * wave) * k_row, nvo = (uint32_t)(kn * kPfBN + 16 * wave) * v_row;
+        auto copy = [&](int c) __attribute__((always_inline)) {   // copy c/2 of the next tile's K rows (c even) or V rows
+            if (c & 1) dma16_buf(rv, vv[c >> 1] + nvo, nl0 + kTileBytes + 4 * (c >> 1) * 256);
+            else dma16_buf(rk, vk[c >> 1] + nko, nl0 + 4 * (c >> 1) * 256);
+        };
         const int cl = __builtin_amdgcn_readfirstlane(class_of(kt));
         const int key0 = kt * kPfBN;
         const bool general =
@@ -592,10 +592,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         for (int t = 0; t < 8; t++) {
             fetch(t + kPfLook);
             sa = MF::run(__builtin_bit_cast(V8, op[t & 7]), qb[t], t == 0 ? f32x16{} : sa);
-            if (do_issue) {   // the next tile's copy c = t/2 of its K rows (t even) or V rows
-                if (t & 1) dma16_buf(nrv, vv[t >> 1], nl0 + kTileBytes + 4 * (t >> 1) * 256);
-                else dma16_buf(nrk, vk[t >> 1], nl0 + 4 * (t >> 1) * 256);
-            }
+            if (do_issue) copy(t);
             __builtin_amdgcn_sched_barrier(0);
         }
         if (general) general_x(sa, key0, cl, (uint32_t)tbits);

@@ -168,11 +168,10 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
     auto voff = [&](const uint32_t (&vd_)[2], int c) __attribute__((always_inline)) {
         return vd_[c & 1] + 4u * (uint32_t)c * v_row;
     };
-    auto tile_rsrc = [&](const char *base, uint64_t avail, uint32_t row, int kt) __attribute__((always_inline)) {
-        const uint32_t off = (uint32_t)(kt * kPfBN + 16 * wave) * row;
-        const uint64_t n = kt < a.n_kt && avail > off ? min(avail - off, (uint64_t)0xFFFFFFFFu) : 0;
-        return buf_rsrc(base + off, (uint32_t)n);
-    };
+    // (one resource for all tiles, as in fa_mfma.hip: a copy's offset is its
+    // place in the tile plus the tile's first row)
+    const i32x4 rk = buf_rsrc(kbase, (uint32_t)min(k_avail, (uint64_t)0xFFFFFFFFu));
+    const i32x4 rv = buf_rsrc(vbase, (uint32_t)min(v_avail, (uint64_t)0xFFFFFFFFu));
     auto next_live = [&](int kt) __attribute__((always_inline)) -> int {
         if constexpr (SM) {
             const int k = max(kt, sm_kt_first);
@@ -189,12 +188,11 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
     int kt = next_live(0);
     if (kt < n_kt) {   // the first live tile's copies go out before Q is loaded
         const uint32_t l0 = lds0 + (uint32_t)(16 * wave) * 256u;
-        const i32x4 rk = tile_rsrc(kbase, k_avail, k_row, kt);
-        const i32x4 rv = tile_rsrc(vbase, v_avail, v_row, kt);
+        const uint32_t row = (uint32_t)(kt * kPfBN + 16 * wave);
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            dma16_buf(rk, koff(kd, kx, c), l0 + 4 * c * 256);
-            dma16_buf(rv, voff(vd, c), l0 + kTileBytes + 4 * c * 256);
+            dma16_buf(rk, koff(kd, kx, c) + row * k_row, l0 + 4 * c * 256);
+            dma16_buf(rv, voff(vd, c) + row * v_row, l0 + kTileBytes + 4 * c * 256);
         }
     }
 
@@ -353,11 +351,7 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
         constexpr int NST = decltype(nst_c)::value;
         const bool do_issue = kn < n_kt;   // uniform
         const uint32_t nl0 = lds0 + NST * kStageBytes + (uint32_t)(16 * wave) * 256u;
-        i32x4 nrk = {0, 0, 0, 0}, nrv = {0, 0, 0, 0};
-        if (do_issue) {
-            nrk = tile_rsrc(kbase, k_avail, k_row, kn);
-            nrv = tile_rsrc(vbase, v_avail, v_row, kn);
-        }
+        const uint32_t nko = (uint32_t)(kn * kPfBN + 16 * wave) * k_row, nvo = (uint32_t)(kn * kPfBN + 16 * wave) * v_row;
         const int cl = __builtin_amdgcn_readfirstlane(class_of(kt));
         const int key0 = kt * kPfBN;
         const bool general =
@@ -399,8 +393,8 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
             fetch(n + kLook);
             qk3(sa, n);
             if (do_issue) {   // copy c = n/2 of the next tile's K rows (n even) or V rows
-                if (n & 1) dma16_buf(nrv, voff(tvd, n >> 1), nl0 + kTileBytes + 4 * (n >> 1) * 256);
-                else dma16_buf(nrk, koff(tkd, tkx, n >> 1), nl0 + 4 * (n >> 1) * 256);
+                if (n & 1) dma16_buf(rv, voff(tvd, n >> 1) + nvo, nl0 + kTileBytes + 4 * (n >> 1) * 256);
+                else dma16_buf(rk, koff(tkd, tkx, n >> 1) + nko, nl0 + 4 * (n >> 1) * 256);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
