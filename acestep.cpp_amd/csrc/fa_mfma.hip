@@ -71,7 +71,7 @@ struct __attribute__((packed, aligned(2))) U64Any {
 // gives such rows.  A 4-key group that would run past key Skv - 1 is read
 // from key Skv - 4 and shifted, so that no load leaves the row.
 template <bool UNAL>
-__global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint8_t *cls) {
+__global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint8_t *cls, uint8_t *cls64) {
     // One workgroup per (key tile, query tile, mask plane).  Each row of the
     // tile (64 keys = 128 B) is read by 16 lanes with 8-byte loads (8-byte
     // aligned rows, or UNAL).  All 8 loads of a
@@ -123,31 +123,47 @@ __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint
         for (int pass = 0; pass < kPfBM / 16; pass++)
             v[pass] = __builtin_bit_cast(u16x4, __builtin_bit_cast(uint64_t, v[pass]) >> sh);
     }
-    bool all_ninf = true, all_zero = true, all_bin = true;
+    bool all_ninf[2] = {true, true}, all_zero[2] = {true, true}, all_bin[2] = {true, true};   // of the two 64-row halves
     uint32_t live = 0;   // bit 4 pass + i: key k + i of row q_lo + r0 + 16 pass is live (0 past Skv)
 #pragma unroll
     for (int pass = 0; pass < kPfBM / 16; pass++) {
+        const int hf = pass / 4;
         const bool row_ok = q_lo + r0 + 16 * pass < a.Sq;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const bool ok = row_ok & (k + i < a.Skv);
             const bool ninf = v[pass][i] == 0xFC00u, zero = (v[pass][i] & 0x7FFFu) == 0;
-            all_ninf &= !ok | ninf;
-            all_zero &= !ok | zero;
-            all_bin &= !ok | ninf | zero;
+            all_ninf[hf] &= !ok | ninf;
+            all_zero[hf] &= !ok | zero;
+            all_bin[hf] &= !ok | ninf | zero;
             live |= (uint32_t)(k + i < a.Skv && !ninf) << (4 * pass + i);
         }
     }
-    // wave votes, then one barrier across the 4 waves
+    // wave votes (3 bits per half), then one barrier across the 4 waves
     __shared__ uint32_t votes[4];
-    const uint64_t bad_ninf = __ballot(!all_ninf), bad_zero = __ballot(!all_zero), bad_bin = __ballot(!all_bin);
-    if ((threadIdx.x & 63) == 0)
-        votes[threadIdx.x >> 6] = (bad_ninf ? 1u : 0u) | (bad_zero ? 2u : 0u) | (bad_bin ? 4u : 0u);
+    uint32_t vote = 0;
+#pragma unroll
+    for (int hf = 0; hf < 2; hf++) {
+        const uint64_t bad_ninf = __ballot(!all_ninf[hf]), bad_zero = __ballot(!all_zero[hf]),
+                       bad_bin = __ballot(!all_bin[hf]);
+        vote |= ((bad_ninf ? 1u : 0u) | (bad_zero ? 2u : 0u) | (bad_bin ? 4u : 0u)) << (4 * hf);
+    }
+    if ((threadIdx.x & 63) == 0) votes[threadIdx.x >> 6] = vote;
     __syncthreads();
-    const uint32_t any = votes[0] | votes[1] | votes[2] | votes[3];
-    const int c = !(any & 1u) ? 0 : (!(any & 2u) ? 1 : (!(any & 4u) && a.tile_bits ? 3 : 2));
-    if (threadIdx.x == 0) cls[((int64_t)plane * a.n_qt + qt) * a.n_kt_pad + kt] = (uint8_t)c;
-    if (c == 3) {   // (uniform) the liveness words of the tile's rows
+    const uint32_t any2 = votes[0] | votes[1] | votes[2] | votes[3];
+    auto class_of = [&](uint32_t any) -> int {
+        return !(any & 1u) ? 0 : (!(any & 2u) ? 1 : (!(any & 4u) && a.tile_bits ? 3 : 2));
+    };
+    const int c = class_of((any2 | any2 >> 4) & 7u), c0 = class_of(any2 & 7u), c1 = class_of(any2 >> 4);
+    if (threadIdx.x == 0) {
+        cls[((int64_t)plane * a.n_qt + qt) * a.n_kt_pad + kt] = (uint8_t)c;
+        if (cls64) {
+            uint8_t *p = cls64 + ((int64_t)plane * 2 * a.n_qt + 2 * qt) * a.n_kt_pad + kt;
+            p[0] = (uint8_t)c0;
+            p[a.n_kt_pad] = (uint8_t)c1;
+        }
+    }
+    if (c == 3 || (cls64 && (c0 == 3 || c1 == 3))) {   // (uniform) the liveness words of the tile's rows
         uint64_t *bits = a.tile_bits + (((int64_t)plane * a.n_qt + qt) * a.n_kt + kt) * kPfBM;
 #pragma unroll
         for (int pass = 0; pass < kPfBM / 16; pass++) {
@@ -760,12 +776,13 @@ fa_prefill_q8q_kernel(const FaArgs a) {
     fa_prefill_body<T_F16, CAP, SM, true, true, false>(a);
 }
 
-hipError_t launch_mask_classify(const FaArgs &a, int n_planes, uint8_t *classes, hipStream_t stream) {
+hipError_t launch_mask_classify(const FaArgs &a, int n_planes, uint8_t *classes, uint8_t *cls64,
+                                hipStream_t stream) {
     // (1D over every tile of the n_planes = m_ne2 * m_ne3 mask planes)
     if (n_planes != a.m_ne2 * a.m_ne3) return hipErrorInvalidValue;
     dim3 grid((uint32_t)a.n_kt * (uint32_t)a.n_qt * (uint32_t)n_planes);
-    if (a.mask_unal) hipLaunchKernelGGL(mask_classify_kernel<true>, grid, dim3(256), 0, stream, a, classes);
-    else hipLaunchKernelGGL(mask_classify_kernel<false>, grid, dim3(256), 0, stream, a, classes);
+    if (a.mask_unal) hipLaunchKernelGGL(mask_classify_kernel<true>, grid, dim3(256), 0, stream, a, classes, cls64);
+    else hipLaunchKernelGGL(mask_classify_kernel<false>, grid, dim3(256), 0, stream, a, classes, cls64);
     return hipGetLastError();
 }
 

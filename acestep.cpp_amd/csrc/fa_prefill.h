@@ -1,5 +1,5 @@
-// fa_prefill.h -- pieces shared by the two MFMA prefill kernels
-// (fa_mfma.hip: 32 queries per wave; fa_wide.hip: 48 queries per wave):
+// fa_prefill.h -- pieces shared by the three MFMA prefill kernels
+// (fa_mfma.hip: 32 queries per wave; fa_wide.hip: 48; fa_narrow.hip: 16):
 // LDS tile geometry, the XCD-aware job order, tile classes held in
 // registers, and cross-lane pair reductions.
 #pragma once
@@ -14,6 +14,7 @@ constexpr int kStageBytes = 2 * kTileBytes;  // K + V
 constexpr int kPfLds = 2 * kStageBytes;      // double buffered: 64 KB
 constexpr uint32_t kXcds = 8;                // MI355X: workgroups go round-robin to 8 XCDs
 constexpr uint32_t kCusPerXcd = 32;          // 256 CUs
+constexpr int64_t kPfCus = 256;
 
 // Job of this workgroup among n_qt * Nh * B (query tile, q head, batch)
 // jobs.  Workgroup ids go round-robin to the XCDs; each XCD gets a

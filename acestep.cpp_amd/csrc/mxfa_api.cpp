@@ -305,6 +305,8 @@ struct Plan {
     bool prefill = false;
     size_t cls_block = 0;   // prefill under a dense mask: tile classes, then (bits_off > 0) liveness words
     size_t bits_off = 0;
+    size_t cls64_off = 0;   // > 0: the classes of 64-query tiles follow the first classes
+    bool narrow = false;    // prefill on the 16-query-per-wave kernel (fa_narrow.hip)
     bool wide = false;   // prefill on the 48-query-per-wave kernel (fa_wide.hip)
     FaArgs args{};
     int ktype = 0;
@@ -523,6 +525,9 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     // (Q8_0 calls keep reading mask values: their prefill instance has no
     // word path)
     const bool bits_fit = mask && !q8 && with_bits <= ws_cap;
+    // the classes of 64-query tiles (fa_narrow.hip), where they fit as well
+    const uint64_t cls64_pf = 2 * cls_pf;
+    const bool cls64_fit = mask && !q8 && ((cls_pf + cls64_pf + 255) & ~255ull) + ((bits_pf + 255) & ~255ull) <= ws_cap;
     pl.prefill = (k->type == MXFA_TYPE_F16 || k->type == MXFA_TYPE_BF16 || q8) && a.Sq >= kPrefillMinSq &&
                  mask_vec_ok && offsets_32 && stage_ok && stage_fits && (!mask || n_kt <= kPfMaxKeyTiles) &&
                  (!a.mask_unal || cls_pf <= ws_cap);
@@ -542,14 +547,22 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         // that the two stay on one kernel (bit-identical outputs).
         // (mask rows without 8-byte alignment: the 32-query kernel, which
         // reads the words of 0 / -inf tiles instead of their values)
-        pl.wide = kPfWide && k->type == MXFA_TYPE_F16 && a.softcap == 0.0f && !a.mask_unal &&
+        // grids that 64-query workgroups fill better (the rule and its
+        // figures: fa_narrow.hip)
+        pl.narrow = !q8 && (!mask || cls64_fit) && fa_narrow_serves(a);
+        a.n_qt_n = pl.narrow ? (a.Sq + kPfNarrowBM - 1) / kPfNarrowBM : 0;
+        pl.wide = !pl.narrow && kPfWide && k->type == MXFA_TYPE_F16 && a.softcap == 0.0f && !a.mask_unal &&
                   ((!mask && a.sm_flags == 0) || n_kt <= kPfWideMaskedMaxKt);
         a.n_qt_w = pl.wide ? (a.Sq + kPfWideBM - 1) / kPfWideBM : 0;
         pl.n_planes = mask ? a.m_ne2 * a.m_ne3 : 0;
         pl.ws_bytes = mask ? (size_t)pl.n_planes * a.n_qt * a.n_kt_pad : 0;
+        if (cls64_fit) {
+            pl.cls64_off = pl.ws_bytes;
+            pl.ws_bytes += (size_t)cls64_pf;
+        }
         if (bits_fit) {
             pl.bits_off = (pl.ws_bytes + 255) & ~(size_t)255;
-            pl.ws_bytes = (size_t)with_bits;
+            pl.ws_bytes = pl.bits_off + (((size_t)bits_pf + 255) & ~(size_t)255);
         }
         pl.cls_block = pl.ws_bytes;
         a.n_splits = 1;
@@ -921,14 +934,17 @@ int run(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const 
                 else classify = true;
             }
             a.tile_class = cls;
+            uint8_t *cls64 = pl.cls64_off ? cls + pl.cls64_off : nullptr;
+            a.tile_class64 = cls64;
             a.tile_bits = pl.bits_off ? (uint64_t *)(cls + pl.bits_off) : nullptr;
             if (classify) {
                 e = timed_launch("mask_classify", stream,
-                                 [&] { return launch_mask_classify(a, pl.n_planes, cls, stream); });
+                                 [&] { return launch_mask_classify(a, pl.n_planes, cls, cls64, stream); });
                 if (e != hipSuccess) return fail(MXFA_ERR_HIP, "mask classify launch: %s", hipGetErrorString(e));
             }
         }
         e = timed_launch("fa_prefill", stream, [&] {
+            if (pl.narrow) return launch_fa_narrow(a, pl.ktype, stream);
             return pl.wide ? launch_fa_wide(a, pl.ktype, stream) : launch_fa_prefill(a, pl.ktype, stream);
         });
         if (e != hipSuccess) return fail(MXFA_ERR_HIP, "prefill launch: %s", hipGetErrorString(e));

@@ -77,6 +77,8 @@ struct FaArgs {
     const uint8_t *tile_class;
     uint64_t *tile_bits;
     int32_t n_qt, n_kt;                   // tiles along Sq and Skv
+    const uint8_t *tile_class64;          // the same classes per 64-query half of a tile (fa_narrow.hip)
+    int32_t n_qt_n;                       // fa_narrow.hip: 64-query tiles along Sq
     int32_t n_qt_w;                       // fa_wide.hip: 192-query tiles along Sq (0: not used)
     int32_t n_kt_pad;                     // class row stride (n_kt rounded up to 4)
     // structured mask (sm_flags == 0: none; then `mask` may hold a dense one)
@@ -338,6 +340,14 @@ __device__ __forceinline__ i32x4 buf_rsrc(const void *base, uint32_t bytes) {
 // MXFA_WAIT_VMCNT before reading the buffer).
 __device__ __forceinline__ void dma16_buf(const i32x4 &rsrc, uint32_t voff, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :
+                 : "s"(lds_addr), "v"(voff), "s"(rsrc)
+                 : "memory", "m0");
+}
+
+// The same with 4 bytes per lane (bytes land at lds_addr + 4*l).
+__device__ __forceinline__ void dma4_buf(const i32x4 &rsrc, uint32_t voff, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
                  :
                  : "s"(lds_addr), "v"(voff), "s"(rsrc)
                  : "memory", "m0");

@@ -27,7 +27,11 @@ constexpr int kPfBN = 64;    // keys per K/V tile
 // a.tile_bits[((plane * n_qt + qt) * n_kt + kt) * kPfBM + row], bit k for key
 // k of the tile (keys past Skv: 0).
 constexpr int kPfMaxKeyTiles = 512;   // class rows held in two registers per lane
-hipError_t launch_mask_classify(const FaArgs &a, int n_planes, uint8_t *classes, hipStream_t stream);
+// With cls64, the class of each 64-query half of a tile goes to
+// cls64[(plane * 2 * n_qt + 2 * qt + half) * n_kt_pad + kt] as well, and the
+// words are written where the tile or either half is of class 3.
+hipError_t launch_mask_classify(const FaArgs &a, int n_planes, uint8_t *classes, uint8_t *cls64,
+                                hipStream_t stream);
 
 // MFMA prefill / DiT kernel.  ktype: T_F16/T_BF16, or T_Q8_0 for K/V
 // staged in F16 by launch_q8_stage (Q, F32, quantised to Q8_0 on load).
@@ -38,6 +42,14 @@ hipError_t launch_fa_prefill(const FaArgs &a, int ktype, hipStream_t stream);
 // (tile classes as for launch_fa_prefill, over kPfBM-query tiles).
 constexpr int kPfWideBM = 192;   // query rows per workgroup (4 waves x 48)
 hipError_t launch_fa_wide(const FaArgs &a, int ktype, hipStream_t stream);
+
+// MFMA prefill with 16 queries per wave (fa_narrow.hip): kPfNarrowBM-query
+// workgroups over a.n_qt_n tiles; F16/BF16 K/V and every mask form of
+// launch_fa_prefill, a dense mask's classes in a.tile_class64.
+// fa_narrow_serves: whether a call's grid is one of those that gain by it.
+constexpr int kPfNarrowBM = 64;
+bool fa_narrow_serves(const FaArgs &a);
+hipError_t launch_fa_narrow(const FaArgs &a, int ktype, hipStream_t stream);
 
 // F16 staging of a prefill over a Q8_0 cache (q8_stage.hip): the Q8_0 K/V
 // rows, dequantised, into contiguous [128, Skv, Nkv, Bk] F16 buffers (the
