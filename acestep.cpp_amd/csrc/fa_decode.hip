@@ -25,9 +25,9 @@
 //       stage (K 4 KB, V 4 KB, the tile's mask 512 B), filled by HBM->LDS
 //       DMA (global_load_lds) NST-1 blocks ahead of the block being
 //       computed, with explicit vmcnt waits; no K/V byte passes through
-//       VGPRs.  The first stages are issued before the live-range scan
-//       returns (they are right whenever the range starts at the split
-//       start, as it does for every live split of a padding mask).
+//       VGPRs.  The first stages are issued first of all, before the
+//       live-range scan (they are right whenever the range starts at the
+//       split start, as it does for every live split of a padding mask).
 //       S^T = K . Q^T with v_mfma_f32_16x16x32_{f16,bf16} (K rows from
 //       LDS, XOR-swizzled); O^T += V^T . P^T with
 //       v_mfma_f32_16x16x16_{f16,bf16}, V^T read with the gfx950 LDS
@@ -85,12 +85,12 @@ struct Tile {
 __device__ __forceinline__ void sm_tile_keys(const FaArgs &a, int b, int rt, int &lo, int &len) {
     const int r0 = rt * 16, nr = min(16, a.M - r0);
     int lo_f, hi_f, lo_l, hi_l;
-    sm_row_range(a, b, r0 / a.G, lo_f, hi_f);
-    sm_row_range(a, b, (r0 + nr - 1) / a.G, lo_l, hi_l);
+    sm_row_range(a, b, div_fast(r0, a.fd_G), lo_f, hi_f);
+    sm_row_range(a, b, div_fast(r0 + nr - 1, a.fd_G), lo_l, hi_l);
     lo = lo_f;
     len = max(0, hi_l - lo_f);
 }
-__device__ __forceinline__ int sm_tile_splits(const FaArgs &a, int len) { return max(1, (len + a.chunk - 1) / a.chunk); }
+__device__ __forceinline__ int sm_tile_splits(const FaArgs &a, int len) { return max(1, div_fast(len + a.chunk - 1, a.fd_chunk)); }
 
 template <int MM>
 __device__ __forceinline__ Tile make_tile(const FaArgs &a) {
@@ -105,8 +105,8 @@ __device__ __forceinline__ Tile make_tile(const FaArgs &a) {
         // j running over the splits of (b, rt) in order, so that every
         // workgroup streams live keys and none waits behind dead ones.
         const int i = (int)blockIdx.x;
-        t.kvh = i % a.Nkv;
-        int j = i / a.Nkv, b = 0, rt = 0;
+        int j = div_fast(i, a.fd_nkv), b = 0, rt = 0;
+        t.kvh = i - j * a.Nkv;
         for (;;) {
             int lo, len;
             sm_tile_keys(a, b, rt, lo, len);
@@ -132,22 +132,23 @@ __device__ __forceinline__ Tile make_tile(const FaArgs &a) {
         const bool first = L < half;
         if (!first) __builtin_amdgcn_s_sleep(32);
         const int Lh = first ? L : L - half;
-        const int stream = Lh / hs;
-        t.split = __builtin_amdgcn_readfirstlane(2 * (Lh % hs) + (first ? 0 : 1));
-        t.kvh = __builtin_amdgcn_readfirstlane((stream % (int)gridDim.y) / a.row_tiles);
-        t.rt = __builtin_amdgcn_readfirstlane((stream % (int)gridDim.y) % a.row_tiles);
-        t.b = __builtin_amdgcn_readfirstlane(stream / (int)gridDim.y);
+        const int stream = div_fast(Lh, a.fd_hs);
+        t.split = __builtin_amdgcn_readfirstlane(2 * (Lh - stream * hs) + (first ? 0 : 1));
+        t.b = __builtin_amdgcn_readfirstlane(div_fast(stream, a.fd_gy));
+        const int y = stream - t.b * (int)gridDim.y;
+        t.kvh = __builtin_amdgcn_readfirstlane(div_fast(y, a.fd_rt));
+        t.rt = __builtin_amdgcn_readfirstlane(y - t.kvh * a.row_tiles);
     } else {
         t.split = blockIdx.x;
-        t.kvh = blockIdx.y / a.row_tiles;
-        t.rt = blockIdx.y % a.row_tiles;
+        t.kvh = div_fast((int)blockIdx.y, a.fd_rt);
+        t.rt = (int)blockIdx.y - t.kvh * a.row_tiles;
         t.b = blockIdx.z;
     }
-    t.bk = t.b / a.rk3;
+    t.bk = div_fast(t.b, a.fd_rk3);
     t.r = t.rt * 16 + t.c16;
     t.row_ok = t.r < a.M;
-    t.iq1 = t.row_ok ? t.r / a.G : 0;
-    t.head = t.kvh * a.G + (t.row_ok ? t.r % a.G : 0);
+    t.iq1 = t.row_ok ? div_fast(t.r, a.fd_G) : 0;
+    t.head = t.kvh * a.G + (t.row_ok ? t.r - t.iq1 * a.G : 0);
     return t;
 }
 
@@ -256,19 +257,17 @@ __device__ __forceinline__ void q_convert8(const QRaw &r, long (&qq)[4], float (
 }
 
 __device__ __forceinline__ const uint16_t *mask_row(const FaArgs &a, int iq1, int head, int b) {
-    return (const uint16_t *)(a.mask + (int64_t)iq1 * a.m_nb1 + (int64_t)(head % a.m_ne2) * a.m_nb2 +
-                              (int64_t)(b % a.m_ne3) * a.m_nb3);
+    return (const uint16_t *)(a.mask + (int64_t)iq1 * a.m_nb1 + (int64_t)mod_fast(head, a.fd_m2, a.m_ne2) * a.m_nb2 +
+                              (int64_t)mod_fast(b, a.fd_m3, a.m_ne3) * a.m_nb3);
 }
 
 // Live key range [lo, hi) of [k0, k1) over the mask rows of the tile's
 // rows (empty when nothing is live).  Called by the whole workgroup.
 // Workgroup-wide [first, last] of the per-thread live ranges -> [lo, hi).
 __device__ void range_reduce(const Tile &t, int first, int last, int *range_lds, int &lo, int &hi) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        first = min(first, __shfl_xor(first, off));
-        last = max(last, __shfl_xor(last, off));
-    }
+    // (first: the maximum of its complement)
+    first = ~wave_max_i(~first);
+    last = wave_max_i(last);
     if (t.lane == 0) {
         range_lds[t.wave] = first;
         range_lds[kDecWaves + t.wave] = last;
@@ -294,14 +293,15 @@ __device__ __forceinline__ ScanRows scan_rows(const FaArgs &a, const Tile &t) {
     ScanRows sr;
     sr.r0 = t.rt * 16;
     const int nr = min(16, a.M - sr.r0);
-    sr.q_first = sr.r0 / a.G;
-    const int q_last = (sr.r0 + nr - 1) / a.G;
+    sr.q_first = div_fast(sr.r0, a.fd_G);
+    const int q_last = div_fast(sr.r0 + nr - 1, a.fd_G);
     sr.n_scan = a.m_ne2 == 1 ? q_last - sr.q_first + 1 : nr;
     return sr;
 }
 __device__ __forceinline__ const uint16_t *scan_row(const FaArgs &a, const Tile &t, const ScanRows &sr, int si) {
-    const int sq1 = a.m_ne2 == 1 ? sr.q_first + si : (sr.r0 + si) / a.G;
-    const int sh = a.m_ne2 == 1 ? 0 : t.kvh * a.G + (sr.r0 + si) % a.G;
+    const int rq = div_fast(sr.r0 + si, a.fd_G);
+    const int sq1 = a.m_ne2 == 1 ? sr.q_first + si : rq;
+    const int sh = a.m_ne2 == 1 ? 0 : t.kvh * a.G + (sr.r0 + si) - rq * a.G;
     return mask_row(a, sq1, sh, t.b);
 }
 
@@ -348,7 +348,7 @@ __device__ __forceinline__ ScanPre scan_issue(const FaArgs &a, const Tile &t, in
     const int n8 = (k1 - k0) >> 3;
     p.one = a.mask_al16 && ((k1 - k0) & 7) == 0 && sr.n_scan * n8 <= 256;   // uniform
     if (p.one && t.tid < sr.n_scan * n8) {
-        const int si = t.tid / n8;
+        const int si = sr.n_scan == 1 ? 0 : t.tid / n8;
         p.k8 = k0 + 8 * (t.tid - si * n8);
         p.mv = *(const u16x8 *)(scan_row(a, t, sr, si) + p.k8);
     }
@@ -376,108 +376,98 @@ __device__ __forceinline__ void st_agent16(float *p, f32x4 v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
 }
 
-__device__ __forceinline__ float ld_dev(const float *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Log-sum-exp merge of the ns partials of the tile's nr rows (run by the
 // last workgroup of the tile; partial row pr0 + r, partial slots a.n_splits
-// apart).  Thread -> dim t.tid % 128 of rows t.tid / 128 + 2j.  The O
-// partials of the first two rows of a thread (every row when nr <= 4, as in
-// decode) are loaded up front together with every (m, l) pair, so the merge
-// waits for one memory round trip; phase A turns (m, l) into weights in
-// LDS, phase B accumulates in split order (larger nr / ns load the rest in
-// batches of 16).
+// apart).  Rows r, r + 4, ... belong to wave r % 4; a wave's lanes are the
+// splits while the weights are formed (every (m, l) pair of a row in one
+// load, the maximum and the sum by DPP) and dim pairs while O is accumulated.
+// With one or two rows (decode at 16 or 8 query heads over 8 KV heads) four
+// or two waves share a row's splits.  The O partials of a wave's first row
+// (up to 32 splits) are loaded together with the (m, l) pairs: one memory
+// round trip.  (Formed by one thread per row, the weights took a serial chain
+// of LDS reads, ~0.17 us a split.  One layer of a replayed decode token at 16 /
+// 8 heads, with the divisions by multiplication: 4000 keys in 64 splits 19.0
+// -> 16.4 us, 1377 + 1290 keys in 24 splits 14.8 -> 13.9 us.)
 constexpr int kMaxSplits = 64;
+constexpr int kWStride = kMaxSplits + 32;   // weights past ns are zero
+__device__ __forceinline__ u32x2 ld_dev2(const float *p) {   // 8-byte aligned
+    return __builtin_bit_cast(u32x2, __hip_atomic_load((const uint64_t *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
 __device__ void merge_splits(const FaArgs &a, const Tile &t, int64_t pr0, int nr, int ns, float *lds) {
-    const int stride = a.n_splits;           // partial slots per row
-    float *wm = lds;                         // [16][kMaxSplits]: m, then weights
-    float *wl = wm + 16 * kMaxSplits;        // [16][kMaxSplits]: l
-    float *Linv = wl + 16 * kMaxSplits;      // [16]
-    const int d = t.tid & (kD - 1);
-    const int rA = t.tid >> 7, rB = rA + 2;
-    // The first 16 partials of rows rA and rB and the first 1024 (m, l)
-    // pairs go out together: one memory round trip.  (The workgroup's LDS
-    // is free here: its own merge data was read before the ticket's
-    // barriers, and a barrier would also wait for these loads.)
-    float pa[16], pb[16];
-    float mv0[4], lv0[4];
-    {
+    const int stride = a.n_splits;                // partial slots per row
+    float *wm = lds;                              // [16][kWStride] weights
+    float *Linv = wm + 16 * kWStride;             // [16]
+    float *red = Linv + 16;                       // [4 waves][128]: shared rows' partial sums
+    const int lane = t.lane, wave = t.wave;
+    const int parts = nr == 1 ? 4 : nr == 2 ? 2 : 1;          // waves per row (uniform)
+    const int ra = parts == 4 ? 0 : parts == 2 ? (wave & 1) : wave;   // this wave's first row
+    const int part = parts == 4 ? wave : parts == 2 ? (wave >> 1) : 0;
+    // (The workgroup's LDS is free here: its own merge data was read before
+    // the ticket's barriers, and a barrier would also wait for these loads.)
+    u32x2 ml[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int i = t.tid + 256 * u;
-            const int r = i / ns, sp = i - r * ns;
-            const float *pm = a.part_ml + ((pr0 + r) * stride + sp) * 2;
-            mv0[u] = i < nr * ns ? ld_dev(pm) : 0.0f;
-            lv0[u] = i < nr * ns ? ld_dev(pm + 1) : 0.0f;
-        }
-        const float *poA = a.part_o + (pr0 + rA) * stride * kD + d;
-        const float *poB = a.part_o + (pr0 + rB) * stride * kD + d;
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-            pa[u] = (rA < nr && u < ns) ? ld_dev(poA + (int64_t)u * kD) : 0.0f;
-            pb[u] = (rB < nr && u < ns) ? ld_dev(poB + (int64_t)u * kD) : 0.0f;
-        }
+    for (int j = 0; j < 4; j++) {
+        const int r = wave + 4 * j;
+        ml[j] = u32x2{0xFF800000u, 0u};   // m = -inf, l = 0
+        if (r < nr && lane < ns) ml[j] = ld_dev2(a.part_ml + ((pr0 + r) * stride + lane) * 2);
     }
-    for (int i0 = 0; i0 < nr * ns; i0 += 256 * 4) {
-        float mv[4], lv[4];
+    // O of row r, splits part + parts * (u0 + u): slots at or past ns read
+    // the last split's (weight zero)
+    u32x2 po[32];
+    auto load_o = [&](int r, int u0) __attribute__((always_inline)) {
+        const float *p = a.part_o + (pr0 + r) * stride * kD + 2 * lane;
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int i = i0 + t.tid + 256 * u;
-            const int r = i / ns, sp = i - r * ns;
-            const float *pm = a.part_ml + ((pr0 + r) * stride + sp) * 2;
-            mv[u] = i0 == 0 ? mv0[u] : (i < nr * ns ? ld_dev(pm) : 0.0f);
-            lv[u] = i0 == 0 ? lv0[u] : (i < nr * ns ? ld_dev(pm + 1) : 0.0f);
+        for (int v = 0; v < 32; v += 8) {
+            if (part + parts * (u0 + v) >= ns) break;   // uniform
+#pragma unroll
+            for (int u = v; u < v + 8; u++) po[u] = ld_dev2(p + (int64_t)min(part + parts * (u0 + u), ns - 1) * kD);
         }
+    };
+    if (ra < nr) load_o(ra, 0);
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int i = i0 + t.tid + 256 * u;
-            if (i < nr * ns) {
-                const int r = i / ns, sp = i - r * ns;
-                wm[r * kMaxSplits + sp] = mv[u];
-                wl[r * kMaxSplits + sp] = lv[u];
+    for (int j = 0; j < 4; j++) {
+        const int r = wave + 4 * j;
+        if (r >= nr) break;   // uniform
+        const float m = __builtin_bit_cast(float, (uint32_t)ml[j][0]), l = __builtin_bit_cast(float, (uint32_t)ml[j][1]);
+        const float mx = wave_max(m);
+        const float f = (m == -INFINITY) ? 0.0f : fast_exp2(m - mx);
+        const float L = wave_sum(f * l);
+        wm[r * kWStride + lane] = f;
+        if (lane < 32) wm[r * kWStride + kMaxSplits + lane] = 0.0f;
+        if (lane == 0) Linv[r] = (L == 0.0f) ? 0.0f : 1.0f / L;
+    }
+    __syncthreads();
+    for (int r = ra; r < nr; r += 4) {   // (parts > 1: one row)
+        float x = 0.0f, y = 0.0f;
+        for (int u0 = 0; part + parts * u0 < ns; u0 += 32) {
+            if (r != ra || u0 != 0) load_o(r, u0);
+#pragma unroll
+            for (int v = 0; v < 32; v += 8) {
+                if (part + parts * (u0 + v) >= ns) break;
+#pragma unroll
+                for (int u = v; u < v + 8; u++) {
+                    const float w = wm[r * kWStride + part + parts * (u0 + u)];
+                    x = fmaf(w, __builtin_bit_cast(float, (uint32_t)po[u][0]), x);
+                    y = fmaf(w, __builtin_bit_cast(float, (uint32_t)po[u][1]), y);
+                }
             }
         }
-    }
-    __syncthreads();
-    if (t.tid < nr) {
-        const int r = t.tid;
-        float ms_all = -INFINITY;
-        for (int sp = 0; sp < ns; sp++) ms_all = fmaxf(ms_all, wm[r * kMaxSplits + sp]);
-        float Lt = 0.0f;
-        for (int sp = 0; sp < ns; sp++) {
-            const float ms = wm[r * kMaxSplits + sp];
-            const float f = (ms == -INFINITY) ? 0.0f : fast_exp2(ms - ms_all);
-            wm[r * kMaxSplits + sp] = f;
-            Lt = fmaf(f, wl[r * kMaxSplits + sp], Lt);
+        if (parts > 1) {   // uniform over the workgroup
+            red[wave * kD + 2 * lane] = x;
+            red[wave * kD + 2 * lane + 1] = y;
+            __syncthreads();
+            if (part != 0) return;
+            for (int p = 1; p < parts; p++) {
+                const int w = parts == 4 ? p : ra + 2 * p;
+                x += red[w * kD + 2 * lane];
+                y += red[w * kD + 2 * lane + 1];
+            }
         }
-        Linv[r] = (Lt == 0.0f) ? 0.0f : 1.0f / Lt;
+        const int rg = t.rt * 16 + r, iq1o = div_fast(rg, a.fd_G), heado = t.kvh * a.G + rg - iq1o * a.G;
+        float *d = a.dst + (((int64_t)t.b * a.Sq + iq1o) * a.Nh + heado) * kD + 2 * lane;
+        d[0] = x * Linv[r];
+        d[1] = y * Linv[r];
     }
-    __syncthreads();
-    // phase B: row r of this thread, the first 16 partials from `pre`
-    auto accum_row = [&](int r, const float (&pre)[16], bool have_pre) {
-        const float *po = a.part_o + (pr0 + r) * stride * kD + d;
-        float acc = 0.0f;
-        for (int s0 = 0; s0 < ns; s0 += 16) {
-            // (the 16 weights are read together, past ns too: a row holds
-            // kMaxSplits of them, and those past ns are not used)
-            float ov[16], wv[16];
-#pragma unroll
-            for (int u = 0; u < 16; u++) wv[u] = wm[r * kMaxSplits + s0 + u];
-#pragma unroll
-            for (int u = 0; u < 16; u++)
-                ov[u] = (s0 == 0 && have_pre) ? pre[u] : (s0 + u < ns ? ld_dev(po + (int64_t)(s0 + u) * kD) : 0.0f);
-#pragma unroll
-            for (int u = 0; u < 16; u++)
-                if (s0 + u < ns) acc = fmaf(wv[u], ov[u], acc);
-        }
-        const int rg = t.rt * 16 + r;
-        const int iq1o = rg / a.G, heado = t.kvh * a.G + rg % a.G;
-        a.dst[(((int64_t)t.b * a.Sq + iq1o) * a.Nh + heado) * kD + d] = acc * Linv[r];
-    };
-    if (rA < nr) accum_row(rA, pa, true);
-    if (rB < nr) accum_row(rB, pb, true);
-    for (int r = rA + 4; r < nr; r += 2) accum_row(r, pa, false);
 }
 
 // Merges the 4 waves' (m, l, O^T) of the tile and writes the output (one
@@ -488,8 +478,7 @@ __device__ void merge_splits(const FaArgs &a, const Tile &t, int64_t pr0, int nr
 // lsum the lane's share of the row sum.
 __device__ void finish_tile(const FaArgs &a, const Tile &t, int ns, const f32x4 (&o)[8], float m2, float lsum,
                             float *lds, int *last_lds) {
-    lsum += __shfl_xor(lsum, 16);
-    lsum += __shfl_xor(lsum, 32);
+    lsum = sum_pair32(sum_pair16(lsum));
     __syncthreads();
     float *mo = lds;                             // [wave][d][16 rows]
     float *mm = mo + kDecWaves * kD * 16;        // [wave][16] max
@@ -530,7 +519,7 @@ __device__ void finish_tile(const FaArgs &a, const Tile &t, int ns, const f32x4 
         for (int w = 0; w < kDecWaves; w++) sacc += fw[w] * mo[(w * kD + dd0 + e) * 16 + rr];
         acc[e] = sacc;
     }
-    const int iq1o = rglob / a.G, heado = t.kvh * a.G + rglob % a.G;
+    const int iq1o = div_fast(rglob, a.fd_G), heado = t.kvh * a.G + rglob - iq1o * a.G;
     float *dp = a.dst + (((int64_t)t.b * a.Sq + iq1o) * a.Nh + heado) * kD + dd0;
     if (ns == 1) {
         if (!out_row) return;
@@ -645,16 +634,12 @@ fa_decode_lds_kernel(const FaArgs a) {
     __shared__ int range_lds[2 * kDecWaves];
     __shared__ int last_lds;
 
+    warm_args();
     const Tile t = make_tile<MM>(a);
     const SplitRange sr = split_range<MM>(a, t);
     if (sr.skip) return;   // past the stream's last split (uniform: no waits, no LDS, no ticket)
-    // the live-range scan's loads go out first (dense mask), then Q's
-    ScanPre scan{};
-    if constexpr (MM == kMaskVec) scan = scan_issue(a, t, sr.k0, sr.k1);
-    const QRaw qraw = q_issue(a, t);
     const int lane = t.lane, c16 = t.c16, g16 = t.g16;
     V8 qb[4];
-    const float slope_l2 = alibi_slope(a, t.head) * kLog2e;
     const char *kbase = a.k + (int64_t)t.kvh * a.k_nb2 + (int64_t)t.bk * a.k_nb3;
     const char *vbase = a.v + (int64_t)t.kvh * a.v_nb2 + (int64_t)t.bk * a.v_nb3;
     const float sl2 = a.scale * kLog2e;
@@ -663,9 +648,8 @@ fa_decode_lds_kernel(const FaArgs a) {
     const int skv4 = (a.Skv + 3) & ~3;
     const int k0 = sr.k0, k1 = sr.k1;
     uint8_t *ring = smem + t.wave * NST * kStBytes;
-    // structured mask: the live keys of this lane's row
-    int rlo = 0, rhi = 0;
-    if constexpr (MM == kMaskStruct) sm_row_range(a, t.b, t.iq1, rlo, rhi);
+    const uint32_t ring0 =
+        __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_void *)smem) + (uint32_t)(t.wave * NST * kStBytes);
 
     // DMA lane geometry.  K/V: instruction j covers keys 4j..4j+3 of the
     // stage, lane -> (key 4j + lane/16, slot lane%16).  Mask: instruction i
@@ -673,42 +657,75 @@ fa_decode_lds_kernel(const FaArgs a) {
     // rows past M read row 0 of the tile (unused).
     const int dkey = lane >> 4, dslot = lane & 15;
     const int mpair = 2 * (lane & 7);
-    const uint16_t *mdma[2] = {nullptr, nullptr};
-    if constexpr (MM == kMaskVec) {
-#pragma unroll
-        for (int i = 0; i < 2; i++) {
-            int rr = t.rt * 16 + 8 * i + (lane >> 3);
-            if (rr >= a.M) rr = t.rt * 16;
-            mdma[i] = mask_row(a, rr / a.G, t.kvh * a.G + rr % a.G, t.b);
+    // Row addresses: key * stride in 32 x 32 -> 64 bits where the strides
+    // fit 32 bits (all but always).  Instruction j's swizzles differ from the
+    // first one's by constants: K chunk (dslot ^ dkey) ^ 4j, V chunk
+    // (dslot ^ 2 dkey) ^ 8(j & 1).
+    const uint32_t kx = 16u * (uint32_t)(dslot ^ dkey), vx = 16u * (uint32_t)(dslot ^ (2 * dkey));
+    const bool far_rows = (((uint64_t)a.k_nb1 | (uint64_t)a.v_nb1) >> 32) != 0;   // uniform
+    auto issue_kv = [&](int kb, int slot) {
+        const uint32_t st = ring0 + (uint32_t)(slot * kStBytes);
+        if (far_rows) {
+#pragma unroll 1
+            for (int j = 0; j < 4; j++) {
+                const int64_t key = min(kb + 4 * j + dkey, a.Skv - 1);
+                dma16_at(kbase + key * a.k_nb1 + (kx ^ (64u * j)), st + kStK + 1024 * j);
+                dma16_at(vbase + key * a.v_nb1 + (vx ^ (128u * (j & 1))), st + kStV + 1024 * j);
+            }
+            return;
         }
-    }
-    auto issue = [&](int kb, int slot) {
-        uint8_t *st = ring + slot * kStBytes;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int kr = 4 * j + dkey;
-            const int key = min(kb + kr, a.Skv - 1);
-            dma16(kbase + (int64_t)key * a.k_nb1 + 16 * (dslot ^ swz_k(kr)), st + kStK + 1024 * j);
-            dma16(vbase + (int64_t)key * a.v_nb1 + 16 * (dslot ^ swz_dv(kr)), st + kStV + 1024 * j);
+            const uint32_t key = (uint32_t)min(kb + 4 * j + dkey, a.Skv - 1);
+            dma16_at(kbase + ((uint64_t)key * (uint32_t)a.k_nb1 + (kx ^ (64u * j))), st + kStK + 1024 * j);
+            dma16_at(vbase + ((uint64_t)key * (uint32_t)a.v_nb1 + (vx ^ (128u * (j & 1)))), st + kStV + 1024 * j);
         }
+    };
+    const uint16_t *mdma[2] = {nullptr, nullptr};
+    auto issue_mask = [&](int kb, int slot) {
         if constexpr (MM == kMaskVec) {
             // key pairs at or past round_up(Skv, 4) (keys >= Skv, never
             // used) re-read the last pair of the row
             const int kp = min(kb + mpair, skv4 - 2);
 #pragma unroll
-            for (int i = 0; i < 2; i++) dma4(mdma[i] + kp, st + kStM + 256 * i);
+            for (int i = 0; i < 2; i++) dma4_at(mdma[i] + kp, ring0 + (uint32_t)(slot * kStBytes + kStM + 256 * i));
         }
+    };
+    auto issue = [&](int kb, int slot) {
+        issue_kv(kb, slot);
+        issue_mask(kb, slot);
     };
 
     // Speculative fill: the first stages of [k0, k1) -- the whole ring -- go
-    // out before the live range is known, so that the wait below (which the
-    // scan needs anyway) does not leave the ring empty behind it.
+    // out before anything else is loaded and before the live range is known,
+    // so that the wait below (which the scan needs anyway) does not leave the
+    // ring empty behind it.  (After the scan's and Q's loads: 0.1-0.4 us a
+    // call slower up to 4000 keys, level beyond.)
     const int kbw_spec = k0 + 16 * t.wave;
     const int nblk_spec = kbw_spec < k1 ? (k1 - kbw_spec + 63) / 64 : 0;
     // (one stage under a dense mask: a split that the scan finds wholly past
     // its sequence's end then wastes one stage of K/V reads, not a ring)
     const int n_spec = min(MM == kMaskVec ? 1 : NST, nblk_spec);
-    for (int s = 0; s < n_spec; s++) issue(kbw_spec + 64 * s, s);
+    for (int s = 0; s < n_spec; s++) issue_kv(kbw_spec + 64 * s, s);
+    // then the live-range scan's loads (dense mask), Q's, and the stage's
+    // mask rows
+    ScanPre scan{};
+    if constexpr (MM == kMaskVec) scan = scan_issue(a, t, k0, k1);
+    const QRaw qraw = q_issue(a, t);
+    if constexpr (MM == kMaskVec) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            int rr = t.rt * 16 + 8 * i + (lane >> 3);
+            if (rr >= a.M) rr = t.rt * 16;
+            const int rq = div_fast(rr, a.fd_G);
+            mdma[i] = mask_row(a, rq, t.kvh * a.G + rr - rq * a.G, t.b);
+        }
+        if (n_spec) issue_mask(kbw_spec, 0);
+    }
+    const float slope_l2 = alibi_slope(a, t.head) * kLog2e;
+    // structured mask: the live keys of this lane's row
+    int rlo = 0, rhi = 0;
+    if constexpr (MM == kMaskStruct) sm_row_range(a, t.b, t.iq1, rlo, rhi);
 
     q_convert16<KT>(a, qraw, qb);
     int lo = k0, hi = k1;
@@ -905,6 +922,7 @@ fa_decode_reg_kernel(const FaArgs a) {
     __shared__ int range_lds[2 * kDecWaves];
     __shared__ int last_lds;
 
+    warm_args();
     const Tile t = make_tile<MM>(a);
     const SplitRange sr = split_range<MM>(a, t);
     if (sr.skip) return;   // past the stream's last split (uniform: no waits, no LDS, no ticket)

@@ -74,22 +74,11 @@ __device__ __forceinline__ uint32_t class_union4(uint32_t x, uint32_t y) {
     return (x & ~m) | (0x02020202u & m);
 }
 
-// Max / sum of a lane's value and the same register of lane l ^ 32 (one
-// v_permlane32_swap) or l ^ 16 (v_permlane16_swap).
+// Max of a lane's value and the same register of lane l ^ 32 (one
+// v_permlane32_swap).
 __device__ __forceinline__ float max_pair32(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
                                                     false, false);
     return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
 }
-__device__ __forceinline__ float sum_pair32(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
-                                                    false, false);
-    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
-}
-__device__ __forceinline__ float sum_pair16(float x) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
-                                                    false, false);
-    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
-}
-
 }  // namespace mxfa

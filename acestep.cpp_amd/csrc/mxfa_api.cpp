@@ -458,6 +458,10 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     a.G = a.Nh / a.Nkv;
     a.rk3 = (int32_t)(q->ne[3] / k->ne[3]);
     a.M = a.Sq * a.G;
+    a.fd_G = fast_div((uint32_t)a.G);
+    a.fd_rk3 = fast_div((uint32_t)a.rk3);
+    a.fd_m2 = fast_div((uint32_t)a.m_ne2);
+    a.fd_m3 = fast_div((uint32_t)a.m_ne3);
     a.scale = p->scale;
     a.softcap = p->logit_softcap;
     a.max_bias = p->max_bias;
@@ -636,6 +640,11 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     }
     a.n_splits = (int32_t)n_splits;
     a.chunk = (int32_t)chunk;
+    a.fd_rt = fast_div((uint32_t)a.row_tiles);
+    a.fd_gy = fast_div((uint32_t)(a.Nkv * a.row_tiles));
+    a.fd_hs = fast_div((uint32_t)std::max<int64_t>(1, n_splits / 2));
+    a.fd_nkv = fast_div((uint32_t)a.Nkv);
+    a.fd_chunk = fast_div((uint32_t)chunk);
     // Paired splits (fa_decode.hip, make_tile): a dense grid of exactly two
     // workgroups per CU whose first half runs ahead of its second; the even
     // split of each pair (first half) takes kDecPairNum/8 of the pair's

@@ -10,6 +10,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace mxfa {
@@ -43,6 +44,23 @@ typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSmCausal = 1, kSmWindow = 2, kSmLengths = 4, kSmDevice = 8;
 constexpr int kSmMaxLen = 64;   // per-batch lengths carried in the arguments
 
+// n / d for 0 <= n < 2^31 by a multiplication: with s = ceil(log2 d) and
+// mul = floor(2^32 (2^s - d) / d) + 1, n / d = (mulhi(n, mul) + n) >> s
+// (Granlund and Montgomery, "Division by invariant integers using
+// multiplication", 1994).  A division by an argument takes the kernels ~150
+// cycles of dependent instructions; their prologues had a dozen ahead of the
+// first load.
+struct FastDiv {
+    uint32_t mul, sh;
+};
+inline FastDiv fast_div(uint32_t d) {
+    uint32_t s = 0;
+    while (s < 32 && ((uint64_t)1 << s) < d) s++;
+    return FastDiv{(uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << s) - d)) / d + 1), s};
+}
+__device__ __forceinline__ int div_fast(int n, FastDiv f) { return (int)((__umulhi((uint32_t)n, f.mul) + (uint32_t)n) >> f.sh); }
+__device__ __forceinline__ int mod_fast(int n, FastDiv f, int d) { return n - div_fast(n, f) * d; }
+
 // Arguments shared by the attention kernels (passed by value).
 struct FaArgs {
     const char *q, *k, *v, *mask;
@@ -53,6 +71,8 @@ struct FaArgs {
     int64_t m_nb1, m_nb2, m_nb3;
     int32_t m_ne2, m_ne3;
     int32_t Sq, Nh, B, Skv, Nkv, G, rk3;  // G = Nh/Nkv, rk3 = B/Bk
+    FastDiv fd_G, fd_rk3, fd_m2, fd_m3;   // dividers of G, rk3, m_ne2, m_ne3
+    FastDiv fd_rt, fd_gy, fd_hs, fd_nkv, fd_chunk;   // decode: row_tiles, Nkv * row_tiles, n_splits / 2, Nkv, chunk
     int32_t M;                            // rows per (b, kv head) = Sq*G
     int32_t row_tiles;                    // decode kernel: ceil(M/16)
     float scale, softcap;                 // softcap == 0: off
@@ -89,6 +109,23 @@ struct FaArgs {
     int32_t sm_len[kSmMaxLen];
 };
 
+// Brings the kernel arguments (all but the structured mask's lengths) into
+// the scalar cache with one dword per 64-byte line, all in flight together.
+// The compiler loads arguments in groups where it needs them, each group a
+// cold miss of its own: three in a row ahead of a decode workgroup's first
+// load.
+__device__ __forceinline__ void warm_args() {
+    typedef const __attribute__((address_space(4))) int32_t karg;
+    karg *p = (karg *)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int kLines = (int)((offsetof(FaArgs, sm_len) + 63) / 64);
+    static_assert(kLines <= 10, "lines listed below");
+    int x[10];
+#pragma unroll
+    for (int i = 0; i < 10; i++) x[i] = p[16 * (i < kLines ? i : kLines - 1)];
+    asm volatile("" ::"s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]), "s"(x[4]), "s"(x[5]), "s"(x[6]), "s"(x[7]),
+                 "s"(x[8]), "s"(x[9]));
+}
+
 // Cross-lane steps at VALU latency (DPP, v_permlane*_swap) instead of LDS
 // crossbar permutes (ds_bpermute, ~100 cycles each).
 template <int CTRL>
@@ -124,6 +161,48 @@ __device__ __forceinline__ float max_half32(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
                                                     false, false);
     return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+
+// sum of x over lanes l and l ^ 32, l ^ 16
+__device__ __forceinline__ float sum_pair32(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
+                                                    false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+__device__ __forceinline__ float sum_pair16(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
+                                                    false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+// max / sum of x over the wave's 64 lanes (the DPP steps of and_rows16, then
+// the row pairs); every lane active, every lane gets the result
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __builtin_bit_cast(float, dpp_u32<CTRL>(__builtin_bit_cast(uint32_t, v)));
+}
+__device__ __forceinline__ float wave_max(float x) {
+    x = fmaxf(x, dpp_f<0xB1>(x));
+    x = fmaxf(x, dpp_f<0x4E>(x));
+    x = fmaxf(x, dpp_f<0x141>(x));
+    x = fmaxf(x, dpp_f<0x140>(x));
+    return max_half32(max_pair16(x));
+}
+__device__ __forceinline__ float wave_sum(float x) {
+    x += dpp_f<0xB1>(x);
+    x += dpp_f<0x4E>(x);
+    x += dpp_f<0x141>(x);
+    x += dpp_f<0x140>(x);
+    return sum_pair32(sum_pair16(x));
+}
+__device__ __forceinline__ int wave_max_i(int x) {
+    x = max(x, (int)dpp_u32<0xB1>((uint32_t)x));
+    x = max(x, (int)dpp_u32<0x4E>((uint32_t)x));
+    x = max(x, (int)dpp_u32<0x141>((uint32_t)x));
+    x = max(x, (int)dpp_u32<0x140>((uint32_t)x));
+    const auto r = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
+    x = max((int)(uint32_t)r[0], (int)(uint32_t)r[1]);
+    const auto q = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
+    return max((int)(uint32_t)q[0], (int)(uint32_t)q[1]);
 }
 
 // Live keys [lo, hi) of query row iq1 of batch b under the structured mask
@@ -293,8 +372,8 @@ typedef __attribute__((address_space(3))) void lds_void;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
-// Direct HBM -> LDS copy of 16 bytes per lane: lane l's bytes land at
-// lds_base + 16*l (lds_base must be the same for the whole wave).
+// Direct HBM -> LDS copy of 16 bytes per lane: lane l's bytes land at LDS
+// address lds_addr + 16*l (lds_addr must be the same for the whole wave).
 //
 // Issued as inline assembly on purpose: the compiler's own wait insertion
 // treats every LDS read after such a copy as a possible alias and drains
@@ -303,21 +382,14 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // buffer.  Compiler-generated waits for other vector loads stay correct: a
 // copy unknown to the compiler only makes them wait longer (counters retire
 // in order).
-__device__ __forceinline__ void dma16(const void *g, void *lds_base) {
-    const uint32_t lds_addr = (uint32_t)(uintptr_t)(lds_void *)lds_base;
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(g)
+__device__ __forceinline__ void dma16_at(const void *g, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(g)
                  : "memory", "m0");
 }
-
-// Direct HBM -> LDS copy of 4 bytes per lane (4-byte aligned source): lane
-// l's bytes land at lds_base + 4*l.  Same contract as dma16.
-__device__ __forceinline__ void dma4(const void *g, void *lds_base) {
-    const uint32_t lds_addr = (uint32_t)(uintptr_t)(lds_void *)lds_base;
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(g)
+// The same with 4 bytes per lane (4-byte aligned source): lane l's bytes
+// land at lds_addr + 4*l.
+__device__ __forceinline__ void dma4_at(const void *g, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" : : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(g)
                  : "memory", "m0");
 }
 
