@@ -90,13 +90,27 @@ constexpr bool kPfWide = MXFA_WIDE != 0;
 // dense causal mask from a window or padding mask, and a structured mask
 // follows the same rule as its dense form).
 constexpr int64_t kPfWideMaskedMaxKt = 4;
-// Workgroups the decode kernel aims for before it splits the KV range.
-// (build option for A/B runs; 512 = two workgroups per CU measured best:
-// 256, 384, 640, 768, 1024 and 2048 were slower on C3 / C5)
-#ifndef MXFA_SPLIT_TARGET
-#define MXFA_SPLIT_TARGET 512
-#endif
-constexpr int64_t kSplitTargetWgs = MXFA_SPLIT_TARGET;
+// Workgroups the decode kernel aims for before it splits the KV range: 512
+// (two per CU) where that leaves every split long enough, then 256, then
+// 128.  Each split costs its dispatch, its start-up and its place in the
+// merge, so short splits lose more than their parallelism gains.  Device time
+// of a call at 32 / 8 heads, splits x keys (us):
+//                      128 workgroups     256               512
+//   F16   1 x 2000     16 x 128  10.1     32 x 64   11.5    32 x 64   11.4
+//         2 x 1000      8 x 128   9.9     16 x 64   10.8    16 x 64   10.7
+//         1 x 4000     16 x 256  12.3     32 x 128  13.0    64 x 64   18.1
+//         2 x 4000      8 x 512  15.5     16 x 256  14.2    32 x 128  17.5
+//         8 x 1000      2 x 512  15.2      4 x 256  12.8     8 x 128  13.5
+//         1 x 8192     16 x 512  16.0     32 x 256  14.9    64 x 128  19.3
+//         8 x 4000      2 x 2048 41.0      4 x 1024 29.9     8 x 512  31.2
+//         8 ragged, 7424 keys    61.6      4 x 1856 36.7     8 x 928  35.1
+//   Q8_0  4 x 2000      4 x 512  17.5      8 x 256  14.1    16 x 128  16.1
+//         4 x 4000      4 x 1024 26.1      8 x 512  18.5    16 x 256  17.1
+//         4 x 8192      4 x 2048 42.6      8 x 1024 26.7    16 x 512  23.2
+constexpr int64_t kSplitTargets[3] = {512, 256, 128};
+constexpr int64_t kSplitMinKeys512 = 768, kSplitMinKeys512Rows = 512, kSplitMinKeys512Sm = 384, kSplitMinKeys512Q8 = 256;
+constexpr int64_t kSplitMinKeys256 = 256;
+constexpr int64_t kSplitFew = 8;   // this few splits may be short at 256 workgroups
 constexpr int kSplitKeyQuantum = 128;  // register kernel: 4 waves x 32 keys
 constexpr int kSplitKeyQuantumLds = 64;  // LDS kernel: 4 waves x 16 keys
 constexpr int64_t kMaxDecodeSplits = 64;   // merge capacity of the decode kernel
@@ -603,6 +617,13 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     const int64_t max_splits = (a.Skv + quantum - 1) / quantum;
     int64_t n_splits = 1, chunk = 0;
     auto round_q = [&](int64_t x) { return (x + quantum - 1) / quantum * quantum; };
+    const int64_t min512 = !lds_kernel ? kSplitMinKeys512Q8 : a.sm_flags && !sm_dev ? kSplitMinKeys512Sm
+                           : a.row_tiles > 1 ? kSplitMinKeys512Rows : kSplitMinKeys512;
+    auto long_enough = [&](int64_t target, int64_t keys, int64_t splits) {
+        if (splits == 1) return true;
+        if (target == 512) return keys >= min512;
+        return target == 128 || keys >= kSplitMinKeys256 || splits <= kSplitFew;
+    };
     if (a.sm_flags && !sm_dev) {
         // Structured mask: every (batch, kv head, row tile) stream covers
         // the keys its rows see; one chunk size for all of them, from the
@@ -620,8 +641,10 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
                 total += len * a.Nkv;
                 max_len = std::max(max_len, len);
             }
-        chunk = round_q(std::max<int64_t>({(total + kSplitTargetWgs - 1) / kSplitTargetWgs,
-                                           (max_len + kMaxDecodeSplits - 1) / kMaxDecodeSplits, 1}));
+        for (int64_t target : kSplitTargets) {
+            chunk = round_q(std::max<int64_t>({(total + target - 1) / target, (max_len + kMaxDecodeSplits - 1) / kMaxDecodeSplits, 1}));
+            if (long_enough(target, chunk, (max_len + chunk - 1) / chunk)) break;
+        }
         // the grid is the list of live splits, (b, rt, split) major, kv head
         // minor, in the order the kernel walks them (each workgroup walks
         // the (b, rt) list to find its split: short lists only)
@@ -633,10 +656,12 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         }
         if (lens.size() <= (size_t)kMaxLiveListTiles) a.dec_live = (int32_t)live;
     } else {
-        if (base < kSplitTargetWgs)
-            n_splits = std::min<int64_t>({max_splits, (kSplitTargetWgs + base - 1) / base, kMaxDecodeSplits});
-        chunk = round_q((a.Skv + n_splits - 1) / n_splits);
-        n_splits = (a.Skv + chunk - 1) / chunk;
+        for (int64_t target : kSplitTargets) {
+            n_splits = std::max<int64_t>(1, std::min<int64_t>({max_splits, target / base, kMaxDecodeSplits}));
+            chunk = round_q((a.Skv + n_splits - 1) / n_splits);
+            n_splits = (a.Skv + chunk - 1) / chunk;
+            if (long_enough(target, chunk, n_splits)) break;
+        }
     }
     a.n_splits = (int32_t)n_splits;
     a.chunk = (int32_t)chunk;
