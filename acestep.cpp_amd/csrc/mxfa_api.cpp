@@ -479,13 +479,15 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     a.scale = p->scale;
     a.softcap = p->logit_softcap;
     a.max_bias = p->max_bias;
-    // ALiBi constants as ggml computes them (per-head slopes).
-    const uint32_t n_head = (uint32_t)a.Nh;
-    a.n_head_log2 = 1u << (uint32_t)std::floor(std::log2((double)n_head));
-    const float m0 = std::pow(2.0f, -(p->max_bias) / (float)a.n_head_log2);
-    const float m1 = std::pow(2.0f, -(p->max_bias / 2.0f) / (float)a.n_head_log2);
-    a.l2m0 = (float)std::log2((double)m0);
-    a.l2m1 = (float)std::log2((double)m1);
+    // ALiBi constants as ggml computes them (per-head slopes); without a
+    // bias every slope is 1.
+    a.n_head_log2 = 1u << (31 - __builtin_clz((uint32_t)a.Nh));
+    if (p->max_bias != 0.0f) {
+        const float m0 = std::pow(2.0f, -(p->max_bias) / (float)a.n_head_log2);
+        const float m1 = std::pow(2.0f, -(p->max_bias / 2.0f) / (float)a.n_head_log2);
+        a.l2m0 = (float)std::log2((double)m0);
+        a.l2m1 = (float)std::log2((double)m1);
+    }
     a.softcap_in = p->logit_softcap != 0.0f ? p->scale / p->logit_softcap : 0.0f;
     pl.ktype = k->type;
 

@@ -54,8 +54,7 @@ struct FastDiv {
     uint32_t mul, sh;
 };
 inline FastDiv fast_div(uint32_t d) {
-    uint32_t s = 0;
-    while (s < 32 && ((uint64_t)1 << s) < d) s++;
+    const uint32_t s = d > 1 ? 32 - (uint32_t)__builtin_clz(d - 1) : 0;
     return FastDiv{(uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << s) - d)) / d + 1), s};
 }
 __device__ __forceinline__ int div_fast(int n, FastDiv f) { return (int)((__umulhi((uint32_t)n, f.mul) + (uint32_t)n) >> f.sh); }

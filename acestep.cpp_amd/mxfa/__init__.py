@@ -21,6 +21,7 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import os
+import struct
 from dataclasses import dataclass
 from typing import Optional
 
@@ -67,6 +68,10 @@ class MxfaTensor(ctypes.Structure):
         ("nb", ctypes.c_size_t * 4),
         ("data", ctypes.c_void_p),
     ]
+
+
+_TENSOR_FIELDS = struct.Struct("=i4x4q4QQ")   # MxfaTensor's layout
+assert _TENSOR_FIELDS.size == ctypes.sizeof(MxfaTensor)
 
 
 class MxfaParams(ctypes.Structure):
@@ -220,6 +225,11 @@ class DeviceView:
 
     def desc(self) -> MxfaTensor:
         t = MxfaTensor()
+        try:   # (one call for all ten fields: 0.5 us, field by field 1.6 us)
+            _TENSOR_FIELDS.pack_into(t, 0, self.type, *self.ne, *self.nb, self.ptr or 0)
+            return t
+        except (struct.error, TypeError):
+            pass   # values that only int() takes, or out of a field's range
         t.type = int(self.type)
         for i in range(4):
             t.ne[i] = int(self.ne[i])
@@ -228,12 +238,24 @@ class DeviceView:
         return t
 
 
+def _current_stream() -> int:
+    """torch's current stream on the current device, as a handle.  (Through
+    the raw getter: 0.4 us, against 2.7 us for the stream object.)"""
+    import torch
+
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch.cuda.current_device())
+
+
 def _descs(q, k, v, mask, dst):
     dq, dk, dv = q.desc(), k.desc(), v.desc()
     dm = mask.desc() if mask is not None else None
     dd = dst.desc() if dst is not None else None
-    ref = lambda d: ctypes.byref(d) if d is not None else None  # noqa: E731
-    return (dq, dk, dv, dm, dd), (ref(dq), ref(dk), ref(dv), ref(dm), ref(dd))
+    byref = ctypes.byref
+    return (dq, dk, dv, dm, dd), (byref(dq), byref(dk), byref(dv), byref(dm) if dm is not None else None,
+                                  byref(dd) if dd is not None else None)
 
 
 def make_params(scale: float, max_bias: float = 0.0, logit_softcap: float = 0.0,
@@ -264,7 +286,7 @@ def flash_attn_ext(q, k, v, mask, scale, max_bias=0.0, logit_softcap=0.0, prec=P
         dst = DeviceView(TYPE_F32, (DV, Nh, Sq, B), (4, 4 * DV, 4 * DV * Nh, 4 * DV * Nh * Sq),
                          out.data_ptr(), out)
     if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _current_stream()
     keep, refs = _descs(q, k, v, mask, dst)
     p = make_params(scale, max_bias, logit_softcap, prec)
     rc = lib.mxfa_flash_attn_ext(refs[0], refs[1], refs[2], refs[3], ctypes.byref(p), refs[4],
@@ -280,12 +302,10 @@ def flash_attn_ext_noalloc(q, k, v, mask, scale, max_bias=0.0, logit_softcap=0.0
     with the split partials, tickets and mask classes in the library's fixed
     per-GPU scratch (no device allocation by the engine; `dst` is allocated
     here with torch when None)."""
-    import torch
-
     if dst is None:
         dst = _out_view(q, v)
     if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _current_stream()
     keep, refs = _descs(q, k, v, mask, dst)
     p = make_params(scale, max_bias, logit_softcap, prec)
     rc = lib.mxfa_flash_attn_ext_noalloc(refs[0], refs[1], refs[2], refs[3], ctypes.byref(p), refs[4],
@@ -302,10 +322,8 @@ def qk_norm_rope(q, k, v, q_norm, k_norm, positions, eps, freq_base, q_out, k_ou
     cache rows.  All arguments are DeviceViews (rows may be None).
     positions=None: no RoPE (DiT cross-attention), and k/v may hold their
     own number of tokens."""
-    import torch
-
     if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _current_stream()
     ds = [t.desc() if t is not None else None for t in (q, k, v, q_norm, k_norm, positions, q_out, k_out, v_out)]
     dr = rows.desc() if rows is not None else None
     p = MxfaNormRopeParams()
@@ -321,10 +339,8 @@ def qk_norm_rope(q, k, v, q_norm, k_norm, positions, eps, freq_base, q_out, k_ou
 def reserve(q, k, v, mask, scale, max_bias=0.0, logit_softcap=0.0, prec=PREC_F32, stream=None) -> None:
     """Grows the engine's workspace for this call's shapes without launching
     anything, so that the call can then be captured into a HIP graph."""
-    import torch
-
     if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _current_stream()
     keep, refs = _descs(q, k, v, mask, None)
     p = make_params(scale, max_bias, logit_softcap, prec)
     rc = lib.mxfa_reserve(refs[0], refs[1], refs[2], refs[3], ctypes.byref(p), ctypes.c_void_p(int(stream)))
@@ -336,10 +352,8 @@ def graph_begin(stream=None) -> None:
     """Starts one graph's computation on `stream` (mxfa_graph_begin): until
     the next call, FA calls on the stream that share a dense mask (same data
     pointer, shape and strides, same Sq and Skv) classify it once."""
-    import torch
-
     if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _current_stream()
     rc = lib.mxfa_graph_begin(ctypes.c_void_p(int(stream)))
     if rc != OK:
         raise MxfaError(rc, last_error())
@@ -348,10 +362,8 @@ def graph_begin(stream=None) -> None:
 def graph_end(stream=None) -> None:
     """Ends the graph begun on `stream` (mxfa_graph_end): FA calls on it
     classify their masks per call again."""
-    import torch
-
     if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _current_stream()
     rc = lib.mxfa_graph_end(ctypes.c_void_p(int(stream)))
     if rc != OK:
         raise MxfaError(rc, last_error())
@@ -381,10 +393,8 @@ def set_rows(dst: DeviceView, src: DeviceView, rows: DeviceView, stream: Optiona
     rows of `src` are converted to dst's type and written, in place, to the
     rows of `dst` that `rows` (I64 / I32) names.  Asynchronous on `stream`
     (default: torch's current stream).  Returns `dst`; raises MxfaError."""
-    import torch
-
     if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _current_stream()
     dd, ds, dr = dst.desc(), src.desc(), rows.desc()
     rc = lib.mxfa_set_rows(ctypes.byref(dd), ctypes.byref(ds), ctypes.byref(dr), ctypes.c_void_p(int(stream)))
     if rc != OK:
@@ -411,12 +421,10 @@ def flash_attn_ext_masked(q, k, v, spec, scale, max_bias=0.0, logit_softcap=0.0,
                           dst: Optional[DeviceView] = None, stream: Optional[int] = None) -> DeviceView:
     """flash_attn_ext with the mask given as metadata (`mask_spec(...)`):
     the result equals flash_attn_ext with the equivalent dense F16 mask."""
-    import torch
-
     if dst is None:
         dst = _out_view(q, v)
     if stream is None:
-        stream = torch.cuda.current_stream().cuda_stream
+        stream = _current_stream()
     keep, refs = _descs(q, k, v, None, dst)
     p = make_params(scale, max_bias, logit_softcap, prec)
     rc = lib.mxfa_flash_attn_ext_masked(refs[0], refs[1], refs[2], ctypes.byref(spec), ctypes.byref(p), refs[4],
