@@ -368,14 +368,6 @@ __device__ __forceinline__ void scan_finish(const FaArgs &a, const Tile &t, cons
     range_reduce(t, first, last, range_lds, lo, hi);
 }
 
-// 16 bytes stored at agent scope: global_store_dwordx4 with sc1, the
-// encoding a relaxed agent-scope atomic store of each element gets on this
-// architecture (written through past the XCD's L2), in one transaction
-// instead of four.  Complete at device scope once vmcnt drains.
-__device__ __forceinline__ void st_agent16(float *p, f32x4 v) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
-}
-
 // Log-sum-exp merge of the ns partials of the tile's nr rows (run by the
 // last workgroup of the tile; partial row pr0 + r, partial slots a.n_splits
 // apart).  Rows r, r + 4, ... belong to wave r % 4; a wave's lanes are the
@@ -390,9 +382,6 @@ __device__ __forceinline__ void st_agent16(float *p, f32x4 v) {
 // -> 16.4 us, 1377 + 1290 keys in 24 splits 14.8 -> 13.9 us.)
 constexpr int kMaxSplits = 64;
 constexpr int kWStride = kMaxSplits + 32;   // weights past ns are zero
-__device__ __forceinline__ u32x2 ld_dev2(const float *p) {   // 8-byte aligned
-    return __builtin_bit_cast(u32x2, __hip_atomic_load((const uint64_t *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
 __device__ void merge_splits(const FaArgs &a, const Tile &t, int64_t pr0, int nr, int ns, float *lds) {
     const int stride = a.n_splits;                // partial slots per row
     float *wm = lds;                              // [16][kWStride] weights

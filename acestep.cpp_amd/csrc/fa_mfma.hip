@@ -189,7 +189,10 @@ __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint
 // SPREAD: the next tile's copies go out one per QK MFMA of the current
 // tile (true), or all before the tile, with Q loaded as whole rows (false:
 // jobs of few key tiles, chosen in launch_fa_prefill).
-template <int T, bool CAP, bool SM, bool QQ8, bool SPREAD, bool UNAL>
+// SPLIT: a job's live tiles are dealt to several workgroups, tile i to part
+// i mod parts (as many parts as keep pf_tiles tiles each); the parts publish
+// (O, m, l) and the job's last one merges them in part order.
+template <int T, bool CAP, bool SM, bool QQ8, bool SPREAD, bool UNAL, bool SPLIT>
 __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     using MF = Mfma32<T>;
     using V8 = typename MF::v8;
@@ -211,7 +214,9 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // that share K/V rows run on one XCD and share its L2.
     int qt, head, b;
     bool second = false;   // the CU's second workgroup of the first pair
-    pf_job(a, a.n_qt, qt, head, b, second);
+    int job = 0, part = 0;
+    if constexpr (SPLIT) pf_unit(a, a.n_qt, job, part, qt, head, b);
+    else pf_job(a, a.n_qt, qt, head, b, second);
     // The two workgroups of a CU's first pair start together, and both would
     // first fetch Q (64 KB in F32) and their first tile.  The second one
     // waits ~2 us (s_sleep 64: 64 x 64 clocks) so that the first pair's
@@ -261,6 +266,21 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     auto class_of = [&](int kt) __attribute__((always_inline)) -> int {
         if constexpr (SM) return (kt * kPfBN >= sm_in_lo && kt * kPfBN + kPfBN <= sm_in_hi) ? 1 : 2;
         else return tc.at(kt);
+    };
+    // this workgroup's tiles: every parts-th live one from the part-th
+    int parts = 1;
+    if constexpr (SPLIT) {
+        const int n_live = SM ? max(sm_kt_end - sm_kt_first, 0) : tc.count(a.n_kt, lane);
+        parts = min(max(div_fast(n_live + a.pf_tiles - 1, a.fd_tiles), 1), a.pf_parts);
+        parts = __builtin_amdgcn_readfirstlane(parts);
+        if (part >= parts) return;   // uniform
+    }
+    auto after = [&](int kt) __attribute__((always_inline)) -> int {   // this workgroup's next tile after kt
+        if constexpr (!SPLIT) return next_live(kt + 1);
+        if constexpr (SM) return kt + parts < sm_kt_end ? kt + parts : a.n_kt;
+        if (!tc.present) return min(kt + parts, a.n_kt);
+        for (int i = 0; i < parts && kt < a.n_kt; i++) kt = tc.next_live(kt + 1, a.n_kt);
+        return kt;
     };
     // Mask rows of this (batch, head) plane through a buffer resource: lane
     // offset qrow * nb1 + 2 * key (32-bit, the host checks the plane size);
@@ -324,6 +344,8 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // The first live tile's copies go out before Q is loaded: the two
     // fetches share one memory latency.
     int kt = next_live(0);
+    if constexpr (SPLIT)
+        for (int i = 0; i < part && kt < n_kt; i++) kt = next_live(kt + 1);
     if (kt < n_kt) issue(kt, std::integral_constant<int, 0>{});
 
     // Q^T operand for the 8 dim-steps of 16: Q[qrow][16t + 8h + e], F32
@@ -705,7 +727,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     int ofree = 1;   // the stage no tile still reads at the end
     uint64_t cbits = load_bits(kt);
     while (kt < n_kt) {
-        int kn = next_live(kt + 1);
+        int kn = after(kt);
         MXFA_WAIT_VMCNT(0);
         __builtin_amdgcn_s_barrier();
         if (!SPREAD && kn < n_kt) issue(kn, st1);
@@ -715,7 +737,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         ofree = 1;
         kt = kn;
         if (kt >= n_kt) break;
-        kn = next_live(kt + 1);
+        kn = after(kt);
         MXFA_WAIT_VMCNT(0);
         __builtin_amdgcn_s_barrier();
         if (!SPREAD && kn < n_kt) issue(kn, st0);
@@ -727,6 +749,71 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     }
 
     lsum = sum_pair32(lsum);
+    if constexpr (SPLIT) {
+        if (parts > 1) {
+            // The decode merge's protocol (fa_decode.hip, finish_tile): agent
+            // stores, a wait for their acknowledgement in every wave, the
+            // barrier, one ticket; the last part reads every partial back
+            // with agent loads.  Partials keep the accumulators' lane layout,
+            // so a lane merges its own 64 values, in part order (the same
+            // bits whichever part comes last).
+            // (The stores are inline assembly, which the compiler's hazard
+            // checks do not look into: the last MFMAs' results are waited
+            // for here, more than the 18 wait states they need.)
+            asm volatile("s_nop 15\n\ts_nop 15" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
+            const int64_t slot = (int64_t)job * a.pf_parts;
+            float *po = a.part_o + (slot + part) * (kPfBM * kD) + 4 * tid;
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    st_agent16(po + (4 * dt + j) * 1024,
+                               f32x4{o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]});
+            st_agent8(a.part_ml + ((slot + part) * 256 + tid) * 2, m2, lsum);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            int *last = (int *)smem;   // (every wave is past its last tile)
+            if (tid == 0)
+                *last = __hip_atomic_fetch_add(&a.tickets[job], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+            __syncthreads();
+            if (!*last) return;
+            if (tid == 0) __hip_atomic_store(&a.tickets[job], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();   // (`last` is read before O is staged over it)
+            float mx = -INFINITY;
+            for (int p0 = 0; p0 < parts; p0 += 4) {
+                u32x2 w[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    w[u] = ld_dev2(a.part_ml + ((slot + min(p0 + u, parts - 1)) * 256 + tid) * 2);
+#pragma unroll
+                for (int u = 0; u < 4; u++) mx = fmaxf(mx, __builtin_bit_cast(float, (uint32_t)w[u][0]));
+            }
+            lsum = 0.0f;
+#pragma unroll
+            for (int dt = 0; dt < 4; dt++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[dt][r] = 0.0f;
+            for (int p = 0; p < parts; p++) {
+                const u32x2 w = ld_dev2(a.part_ml + ((slot + p) * 256 + tid) * 2);
+                const float *pp = a.part_o + (slot + p) * (kPfBM * kD) + 4 * tid;
+                u32x2 v[32];
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    v[2 * i] = ld_dev2(pp + i * 1024);
+                    v[2 * i + 1] = ld_dev2(pp + i * 1024 + 2);
+                }
+                const float m = __builtin_bit_cast(float, (uint32_t)w[0]);
+                const float f = m == -INFINITY ? 0.0f : fast_exp2(m - mx);
+                lsum = fmaf(f, __builtin_bit_cast(float, (uint32_t)w[1]), lsum);
+#pragma unroll
+                for (int i = 0; i < 32; i++)
+#pragma unroll
+                    for (int e = 0; e < 2; e++)
+                        o[i / 8][2 * (i % 8) + e] =
+                            fmaf(f, __builtin_bit_cast(float, (uint32_t)v[i][e]), o[i / 8][2 * (i % 8) + e]);
+            }
+        }
+    }
     const float inv = (lsum == 0.0f) ? 0.0f : 1.0f / lsum;
     // O leaves as whole rows through the stage the last tile did not read
     // (every wave was past its last read at that tile's barrier, and no
@@ -763,17 +850,17 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     }
 }
 
-template <int T, bool CAP, bool SM, bool SPREAD, bool UNAL>
+template <int T, bool CAP, bool SM, bool SPREAD, bool UNAL, bool SPLIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 fa_prefill_kernel(const FaArgs a) {
-    fa_prefill_body<T, CAP, SM, false, SPREAD, UNAL>(a);
+    fa_prefill_body<T, CAP, SM, false, SPREAD, UNAL, SPLIT>(a);
 }
 
 // Prefill over a Q8_0 cache: K/V rows staged in F16, Q quantised on load.
-template <bool CAP, bool SM>
+template <bool CAP, bool SM, bool SPLIT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 fa_prefill_q8q_kernel(const FaArgs a) {
-    fa_prefill_body<T_F16, CAP, SM, true, true, false>(a);
+    fa_prefill_body<T_F16, CAP, SM, true, true, false, SPLIT>(a);
 }
 
 hipError_t launch_mask_classify(const FaArgs &a, int n_planes, uint8_t *classes, uint8_t *cls64,
@@ -788,13 +875,23 @@ hipError_t launch_mask_classify(const FaArgs &a, int n_planes, uint8_t *classes,
 
 template <int KT, bool CAP, bool SM, bool UNAL>
 static hipError_t launch_pf(const FaArgs &a, dim3 grid, bool spread, hipStream_t stream) {
+    if constexpr (!CAP) {
+        if (a.pf_parts > 0) {
+            grid.x *= (uint32_t)a.pf_parts;
+            if constexpr (KT == T_Q8_0)
+                hipLaunchKernelGGL((fa_prefill_q8q_kernel<CAP, SM, true>), grid, dim3(256), kPfLds, stream, a);
+            else
+                hipLaunchKernelGGL((fa_prefill_kernel<KT, CAP, SM, true, UNAL, true>), grid, dim3(256), kPfLds, stream, a);
+            return hipGetLastError();
+        }
+    }
     if constexpr (KT == T_Q8_0) {
         if constexpr (UNAL) return hipErrorInvalidValue;   // (the host keeps those on the decode kernel)
-        else hipLaunchKernelGGL((fa_prefill_q8q_kernel<CAP, SM>), grid, dim3(256), kPfLds, stream, a);
+        else hipLaunchKernelGGL((fa_prefill_q8q_kernel<CAP, SM, false>), grid, dim3(256), kPfLds, stream, a);
     } else if (spread)
-        hipLaunchKernelGGL((fa_prefill_kernel<KT, CAP, SM, true, UNAL>), grid, dim3(256), kPfLds, stream, a);
+        hipLaunchKernelGGL((fa_prefill_kernel<KT, CAP, SM, true, UNAL, false>), grid, dim3(256), kPfLds, stream, a);
     else
-        hipLaunchKernelGGL((fa_prefill_kernel<KT, CAP, SM, false, UNAL>), grid, dim3(256), kPfLds, stream, a);
+        hipLaunchKernelGGL((fa_prefill_kernel<KT, CAP, SM, false, UNAL, false>), grid, dim3(256), kPfLds, stream, a);
     return hipGetLastError();
 }
 

@@ -43,6 +43,22 @@ __device__ __forceinline__ void pf_job(const FaArgs &a, int n_qt, int &qt, int &
     second = rnd == 1 && n_x >= 2 * kCusPerXcd;
 }
 
+// The same for a key-split grid of n_qt * Nh * B * a.pf_parts workgroups: the
+// parts of a job are neighbours on one XCD, jobs in pf_job's order.
+__device__ __forceinline__ void pf_unit(const FaArgs &a, int n_qt, int &job, int &part, int &qt, int &head, int &b) {
+    const uint32_t L = __builtin_amdgcn_workgroup_id_x();
+    const uint32_t N = (uint32_t)(n_qt * a.Nh * a.B) * (uint32_t)a.pf_parts;
+    const uint32_t nq = N / kXcds, nr = N % kXcds, x = L % kXcds;
+    const int U = (int)(x * nq + min(x, nr) + L / kXcds);
+    job = __builtin_amdgcn_readfirstlane(div_fast(U, a.fd_parts));
+    part = __builtin_amdgcn_readfirstlane(U - job * a.pf_parts);
+    const uint32_t per_u = (uint32_t)(a.G * n_qt), J = (uint32_t)job;
+    const uint32_t u = J / per_u, r = J % per_u;
+    qt = __builtin_amdgcn_readfirstlane(n_qt - 1 - (int)(r / (uint32_t)a.G));
+    b = __builtin_amdgcn_readfirstlane((int)(u / (uint32_t)a.Nkv));
+    head = __builtin_amdgcn_readfirstlane((int)(u % (uint32_t)a.Nkv) * a.G + (int)(r % (uint32_t)a.G));
+}
+
 // Tile classes of one (plane, query tile) row live in registers: lane l
 // holds the class bytes of key tiles 4l..4l+3 (w0: tiles < 256, w1: tiles
 // 256..511), read with v_readlane (uniform, no memory wait in the loop).
@@ -54,6 +70,17 @@ struct TileClasses {
         const uint32_t w = kt < 256 ? __builtin_amdgcn_readlane(w0, (kt >> 2) & 63)
                                     : __builtin_amdgcn_readlane(w1, ((kt - 256) >> 2) & 63);
         return (int)((w >> (8 * (kt & 3))) & 0xFFu);
+    }
+    // live tiles among the first n (every lane active)
+    __device__ __forceinline__ int count(int n, int lane) const {
+        if (!present) return n;
+        int c = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(4 * lane + i < n && ((w0 >> (8 * i)) & 0xFFu)));
+            c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(256 + 4 * lane + i < n && ((w1 >> (8 * i)) & 0xFFu)));
+        }
+        return c;
     }
     // (readfirstlane: the result is wave-uniform, and the compiler must
     // know it to keep the tile loop on scalar branches)

@@ -90,6 +90,22 @@ constexpr bool kPfWide = MXFA_WIDE != 0;
 // dense causal mask from a window or padding mask, and a structured mask
 // follows the same rule as its dense form).
 constexpr int64_t kPfWideMaskedMaxKt = 4;
+// Key-split prefill.  A part costs its start-up, its partial's way out and
+// back (64 KB) and its place in the merge, ~5 us in all, against ~1 us a tile:
+// worth it while the chip has CUs to spare and a row has tiles to share.
+// Measured per call against the unsplit kernels (fa_narrow.hip for F16/BF16),
+// dense causal masks:
+//   jobs x tiles   split                jobs x tiles   split
+//   16 x 28        30.0 (36.1) us       64 x 72        48.5 (97.9) us
+//   32 x 28 BF16   34.9 (45.1)          96 x 20        29.8 (31.9)
+//   32 x 64        42.6 (87.6)          96 x 68        62.2 (96.2)
+//   48 x 20        29.2 (28.1)         128 x 32        39.7 (51.4)
+//   48 x 32        32.5 (45.6)         128 x 80        70.8 (125.0)
+//   64 x 16 BF16   30.4 (28.4)          96 x 24 Q8_0   42.8 (47.2)
+// Grids past half the CUs gain nothing: 288 jobs x 17 tiles BF16 in three
+// parts 52.1 (48.1), 256 x 24 Q8_0 in two 52.1 (52.3).
+constexpr int64_t kPfSplitMinKt = 24, kPfSplitMinKtQ8 = 20;
+constexpr int64_t kPfSplitTiles = 8;   // 4: 48.2 against 43.1 us on 16 x 68; 12: level or slower
 // Workgroups the decode kernel aims for before it splits the KV range: 512
 // (two per CU) where that leaves every split long enough, then 256, then
 // 128.  Each split costs its dispatch, its start-up and its place in the
@@ -320,6 +336,7 @@ struct Plan {
     size_t cls_block = 0;   // prefill under a dense mask: tile classes, then (bits_off > 0) liveness words
     size_t bits_off = 0;
     size_t cls64_off = 0;   // > 0: the classes of 64-query tiles follow the first classes
+    size_t part_off = 0;    // key-split prefill: partials after the classes
     bool narrow = false;    // prefill on the 16-query-per-wave kernel (fa_narrow.hip)
     bool wide = false;   // prefill on the 48-query-per-wave kernel (fa_wide.hip)
     FaArgs args{};
@@ -428,9 +445,11 @@ int check_spec(const mxfa_mask_spec *sm, const mxfa_tensor *q) {
 // ws_cap: workspace bytes the call may use (the allocation-free entry
 // point's fixed scratch); a prompt over a Q8_0 cache whose F16 staging does
 // not fit takes the decode kernel instead, which stages nothing.
+// allow_split: whether a prefill may split its jobs' keys (partials and
+// tickets in the workspace).
 void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const mxfa_tensor *mask,
                const mxfa_params *p, mxfa_tensor *dst, Plan &pl, const mxfa_mask_spec *sm = nullptr,
-               size_t ws_cap = SIZE_MAX) {
+               size_t ws_cap = SIZE_MAX, bool allow_split = true) {
     FaArgs &a = pl.args;
     const bool sm_dev = sm && (sm->flags & MXFA_MASK_DEVICE);
     if (sm && (sm->flags & ~MXFA_MASK_DEVICE)) {
@@ -569,9 +588,21 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         // reads the words of 0 / -inf tiles instead of their values)
         // grids that 64-query workgroups fill better (the rule and its
         // figures: fa_narrow.hip)
-        pl.narrow = !q8 && (!mask || cls64_fit) && fa_narrow_serves(a);
+        // Few jobs over many key tiles: the tiles of a job dealt to several
+        // workgroups (fa_mfma.hip, SPLIT), as many as fill the chip once, of
+        // at least kPfSplitTiles tiles each.
+        const int64_t jobs = (int64_t)a.n_qt * a.Nh * a.B;
+        int64_t split = 0;
+        if (allow_split && a.softcap == 0.0f && n_kt >= (q8 ? kPfSplitMinKtQ8 : kPfSplitMinKt) && 2 * jobs <= kDecCus) {
+            split = std::min<int64_t>({kDecCus / jobs, n_kt / kPfSplitTiles, kPfMaxParts});
+            const uint64_t other = with_bits + cls_pf * 2 + (q8 ? 512ull * (uint64_t)n_kv_rows : 0) + 1024;
+            if (other + (uint64_t)(jobs * split) * kPfPartBytes > ws_cap) split = 0;
+        }
+        // grids that 64-query workgroups fill better (the rule and its
+        // figures: fa_narrow.hip)
+        pl.narrow = !split && !q8 && (!mask || cls64_fit) && fa_narrow_serves(a);
         a.n_qt_n = pl.narrow ? (a.Sq + kPfNarrowBM - 1) / kPfNarrowBM : 0;
-        pl.wide = !pl.narrow && kPfWide && k->type == MXFA_TYPE_F16 && a.softcap == 0.0f && !a.mask_unal &&
+        pl.wide = !split && !pl.narrow && kPfWide && k->type == MXFA_TYPE_F16 && a.softcap == 0.0f && !a.mask_unal &&
                   ((!mask && a.sm_flags == 0) || n_kt <= kPfWideMaskedMaxKt);
         a.n_qt_w = pl.wide ? (a.Sq + kPfWideBM - 1) / kPfWideBM : 0;
         pl.n_planes = mask ? a.m_ne2 * a.m_ne3 : 0;
@@ -587,6 +618,15 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         pl.cls_block = pl.ws_bytes;
         a.n_splits = 1;
         a.chunk = a.Skv;
+        if (split) {
+            a.pf_tiles = (int32_t)((n_kt + split - 1) / split);
+            a.pf_parts = (int32_t)((n_kt + a.pf_tiles - 1) / a.pf_tiles);
+            a.fd_tiles = fast_div((uint32_t)a.pf_tiles);
+            a.fd_parts = fast_div((uint32_t)a.pf_parts);
+            pl.n_tickets = jobs;
+            pl.part_off = (pl.ws_bytes + 255) & ~(size_t)255;
+            pl.ws_bytes = pl.part_off + (size_t)(jobs * a.pf_parts) * kPfPartBytes;
+        }
         if (q8) {
             Q8StageArgs &st = pl.stage;
             st.k = a.k; st.v = a.v;
@@ -931,11 +971,17 @@ int run(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const 
         tickets = fixed->tickets;
     } else {
         int rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
-        if (rc != MXFA_OK && pl.prefill && pl.args.mask_unal) {
-            // (the workspace cannot grow, for instance under capture: such
-            // a mask needs none on the decode kernel)
+        // A workspace that cannot grow (under capture, or out of memory)
+        // leaves a key-split prefill to its unsplit form and a mask of odd
+        // rows to the decode kernel, which need less of it or none.
+        if (rc != MXFA_OK && pl.args.pf_parts > 0) {
             pl = Plan{};
-            make_plan(q, k, v, mask, params, dst, pl, sm, 0);
+            make_plan(q, k, v, mask, params, dst, pl, sm, SIZE_MAX, false);
+            rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
+        }
+        if (rc != MXFA_OK && pl.prefill && pl.args.mask_unal) {
+            pl = Plan{};
+            make_plan(q, k, v, mask, params, dst, pl, sm, 0, false);
             rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
         }
         if (rc != MXFA_OK) return rc;
@@ -945,6 +991,11 @@ int run(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const 
     FaArgs &a = pl.args;
     hipError_t e;
     if (pl.prefill) {
+        if (a.pf_parts > 0) {
+            a.part_o = (float *)((char *)ws + pl.part_off);
+            a.part_ml = a.part_o + (size_t)pl.n_tickets * a.pf_parts * (kPfBM * kD);
+            a.tickets = tickets;
+        }
         if (pl.q8_stage) {
             char *base = (char *)ws + pl.stage_off;
             Q8StageArgs &st = pl.stage;

@@ -97,6 +97,8 @@ struct FaArgs {
     uint64_t *tile_bits;
     int32_t n_qt, n_kt;                   // tiles along Sq and Skv
     const uint8_t *tile_class64;          // the same classes per 64-query half of a tile (fa_narrow.hip)
+    int32_t pf_parts, pf_tiles;           // fa_mfma.hip: key split, workgroups per job (0: none), live tiles per part
+    FastDiv fd_parts, fd_tiles;
     int32_t n_qt_n;                       // fa_narrow.hip: 64-query tiles along Sq
     int32_t n_qt_w;                       // fa_wide.hip: 192-query tiles along Sq (0: not used)
     int32_t n_kt_pad;                     // class row stride (n_kt rounded up to 4)
@@ -422,6 +424,29 @@ __device__ __forceinline__ void dma4_buf(const i32x4 &rsrc, uint32_t voff, uint3
                  :
                  : "s"(lds_addr), "v"(voff), "s"(rsrc)
                  : "memory", "m0");
+}
+
+// 16 bytes stored at agent scope: global_store_dwordx4 with sc1, the
+// encoding a relaxed agent-scope atomic store of each element gets on this
+// architecture (written through past the XCD's L2), in one transaction
+// instead of four.  Complete at device scope once vmcnt drains.
+// The s_nop belongs to the store: a store of more than 8 bytes may still be
+// reading its data registers when the next instruction writes them (one wait
+// state, which the compiler keeps for its own stores but not behind inline
+// assembly; without it, lanes 12-15 and 28-31 stored the address arithmetic
+// that followed).
+__device__ __forceinline__ void st_agent16(float *p, f32x4 v) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+}
+
+__device__ __forceinline__ void st_agent8(float *p, float x, float y) {   // 8-byte aligned
+    __hip_atomic_store((uint64_t *)p, ((uint64_t)__builtin_bit_cast(uint32_t, y) << 32) | __builtin_bit_cast(uint32_t, x),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// 8 bytes (8-byte aligned) loaded at agent scope, from the coherence point.
+__device__ __forceinline__ u32x2 ld_dev2(const float *p) {
+    return __builtin_bit_cast(u32x2, __hip_atomic_load((const uint64_t *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
 // LDS transpose read of four 16-bit values.  Within each group of 16 lanes,

@@ -37,6 +37,12 @@ hipError_t launch_mask_classify(const FaArgs &a, int n_planes, uint8_t *classes,
 // staged in F16 by launch_q8_stage (Q, F32, quantised to Q8_0 on load).
 hipError_t launch_fa_prefill(const FaArgs &a, int ktype, hipStream_t stream);
 
+// Key-split calls (a.pf_parts > 0): at most kPfMaxParts workgroups per job,
+// each with a partial of kPfPartBytes (O, then (m, l) of every lane) in
+// a.part_o / a.part_ml, and one ticket per job in a.tickets.
+constexpr int64_t kPfMaxParts = 16;
+constexpr size_t kPfPartBytes = (size_t)kPfBM * kD * 4 + 256 * 8;
+
 // MFMA prefill with 48 queries per wave (fa_wide.hip): kPfWideBM-query
 // workgroups over a.n_qt_w tiles; F16 K/V, no softcap, dense mask or none
 // (tile classes as for launch_fa_prefill, over kPfBM-query tiles).
