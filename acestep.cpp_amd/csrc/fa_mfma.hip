@@ -84,12 +84,13 @@ __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint
     // x-th contiguous eighth of the tiles: neighbouring key tiles of a row
     // share the 128-byte lines their row pieces straddle (rows whose length
     // is not a multiple of 128 bytes), and fetch them into one L2.
+    warm_args();
     const uint32_t n_tiles = (uint32_t)a.n_kt * (uint32_t)a.n_qt * (uint32_t)(a.m_ne2 * a.m_ne3);
     const uint32_t L = blockIdx.x, x = L % kXcds, per = n_tiles / kXcds, rem = n_tiles % kXcds;
     const uint32_t T = x * per + min(x, rem) + L / kXcds;
-    const int kt = (int)(T % (uint32_t)a.n_kt), qt = (int)((T / (uint32_t)a.n_kt) % (uint32_t)a.n_qt);
-    const int plane = (int)(T / ((uint32_t)a.n_kt * (uint32_t)a.n_qt));
-    const int m2i = plane % a.m_ne2, m3i = plane / a.m_ne2;
+    const int row = div_fast((int)T, a.fd_kt), kt = (int)T - row * a.n_kt;
+    const int plane = div_fast(row, a.fd_qt), qt = row - plane * a.n_qt;
+    const int m3i = div_fast(plane, a.fd_m2), m2i = plane - m3i * a.m_ne2;
     // (the plane base is uniform; readfirstlane lets the compiler know, so
     // the buffer loads need no waterfall loop.  readfirstlane returns a
     // signed int: each half is taken as uint32_t before it is widened, or a
@@ -203,6 +204,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     constexpr bool kBits = !SM && !QQ8;
 
     // (work-item / group ids through the intrinsics: always inline, scalar)
+    warm_args();
     const int tid = (int)__builtin_amdgcn_workitem_id_x();
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -212,11 +214,11 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // (batch, kv head), then by query tile from the last (longest under a
     // causal mask) down, then by q head within the GQA group: the q tiles
     // that share K/V rows run on one XCD and share its L2.
-    int qt, head, b;
+    int qt, head, kvh, b;
     bool second = false;   // the CU's second workgroup of the first pair
     int job = 0, part = 0;
-    if constexpr (SPLIT) pf_unit(a, a.n_qt, job, part, qt, head, b);
-    else pf_job(a, a.n_qt, qt, head, b, second);
+    if constexpr (SPLIT) pf_unit(a, a.n_qt, job, part, qt, head, kvh, b);
+    else pf_job(a, a.n_qt, qt, head, kvh, b, second);
     // The two workgroups of a CU's first pair start together, and both would
     // first fetch Q (64 KB in F32) and their first tile.  The second one
     // waits ~2 us (s_sleep 64: 64 x 64 clocks) so that the first pair's
@@ -225,7 +227,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // each CU's two workgroups stay out of phase between loading and
     // computing.  Measured: C2 55.0 -> 53.9 us, C4 cross 37.3 -> 34.9 us.
     if (second) __builtin_amdgcn_s_sleep(64);
-    const int kvh = head / a.G, bk = b / a.rk3;
+    const int bk = div_fast(b, a.fd_rk3);
     const int qrow = qt * kPfBM + wave * 32 + l32;
     const bool row_ok = qrow < a.Sq;
     const int qrow_c = row_ok ? qrow : a.Sq - 1;
@@ -246,7 +248,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         sm_in_hi = __builtin_amdgcn_readfirstlane(hi_f);
         sm_row_range(a, b, qrow_c, row_lo, row_hi);
     }
-    const int plane = a.mask ? (b % a.m_ne3) * a.m_ne2 + head % a.m_ne2 : 0;
+    const int plane = a.mask ? mod_fast(b, a.fd_m3, a.m_ne3) * a.m_ne2 + mod_fast(head, a.fd_m2, a.m_ne2) : 0;
     TileClasses tc{0u, 0u, !SM && a.tile_class != nullptr};
     if (tc.present) {
         const uint32_t *row = (const uint32_t *)(a.tile_class + ((int64_t)plane * a.n_qt + qt) * a.n_kt_pad);
@@ -286,7 +288,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // offset qrow * nb1 + 2 * key (32-bit, the host checks the plane size);
     // reads past the plane return zeros, so 4-key groups at the row end need
     // no clamp (keys past Skv are masked anyway).
-    const char *mplane = a.mask ? a.mask + (int64_t)(head % a.m_ne2) * a.m_nb2 + (int64_t)(b % a.m_ne3) * a.m_nb3
+    const char *mplane = a.mask ? a.mask + (int64_t)(mod_fast(head, a.fd_m2, a.m_ne2)) * a.m_nb2 + (int64_t)mod_fast(b, a.fd_m3, a.m_ne3) * a.m_nb3
                                 : a.q;
     const __amdgpu_buffer_rsrc_t mrs =
         __builtin_amdgcn_make_buffer_rsrc((void *)mplane, (short)0, a.mask ? (int)a.m_plane_bytes : 0, 0x00020000);

@@ -53,18 +53,19 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
     static_assert(kD == 128, "kernel is written for D = 128");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
+    warm_args();
     const int tid = (int)__builtin_amdgcn_workitem_id_x();
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n16 = lane & 15, g = lane >> 4;
-    int qt, head, b;
+    int qt, head, kvh, b;
     bool second = false;   // (no staggered start: measured level)
-    pf_job(a, a.n_qt_n, qt, head, b, second);
-    const int kvh = head / a.G, bk = b / a.rk3;
+    pf_job(a, a.n_qt_n, qt, head, kvh, b, second);
+    const int bk = div_fast(b, a.fd_rk3);
     const int q0w = qt * kPfNarrowBM + wave * 16;
     const int qrow = min(q0w + n16, a.Sq - 1);   // rows past Sq: the last row (not stored)
 
-    const int plane = a.mask ? (b % a.m_ne3) * a.m_ne2 + head % a.m_ne2 : 0;
+    const int plane = a.mask ? mod_fast(b, a.fd_m3, a.m_ne3) * a.m_ne2 + mod_fast(head, a.fd_m2, a.m_ne2) : 0;
     TileClasses tc{0u, 0u, DENSE};
     if constexpr (DENSE) {
         const uint32_t *row = (const uint32_t *)(a.tile_class64 + ((int64_t)plane * 2 * a.n_qt + qt) * a.n_kt_pad);
@@ -97,7 +98,7 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
         if constexpr (SM) return (kt * kPfBN >= sm_in_lo && kt * kPfBN + kPfBN <= sm_in_hi) ? 1 : 2;
         else return tc.at(kt);
     };
-    const char *mplane = DENSE ? a.mask + (int64_t)(head % a.m_ne2) * a.m_nb2 + (int64_t)(b % a.m_ne3) * a.m_nb3 : a.q;
+    const char *mplane = DENSE ? a.mask + (int64_t)(mod_fast(head, a.fd_m2, a.m_ne2)) * a.m_nb2 + (int64_t)mod_fast(b, a.fd_m3, a.m_ne3) * a.m_nb3 : a.q;
     const __amdgpu_buffer_rsrc_t mrs =
         __builtin_amdgcn_make_buffer_rsrc((void *)mplane, (short)0, DENSE ? (int)a.m_plane_bytes : 0, 0x00020000);
     const uint32_t mrow_off = (uint32_t)qrow * (uint32_t)a.m_nb1 + 8u * (uint32_t)g;

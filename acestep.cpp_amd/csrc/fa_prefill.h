@@ -26,7 +26,16 @@ constexpr int64_t kPfCus = 256;
 // odd rounds run reversed and a CU pairs a long causal tile with a short
 // one.  `second`: the workgroup is the CU's second of the first pair (every
 // CU of the XCD holds a pair).
-__device__ __forceinline__ void pf_job(const FaArgs &a, int n_qt, int &qt, int &head, int &b, bool &second) {
+__device__ __forceinline__ void pf_place(const FaArgs &a, int n_qt, int J, int &qt, int &head, int &kvh, int &b) {
+    // job J: (batch, kv head) major, then the query tile from the last one
+    // down, then the q head within the group
+    const int u = div_fast(J, a.fd_unit), r = J - u * a.G * n_qt, t = div_fast(r, a.fd_G);
+    qt = __builtin_amdgcn_readfirstlane(n_qt - 1 - t);
+    b = __builtin_amdgcn_readfirstlane(div_fast(u, a.fd_nkv));
+    kvh = __builtin_amdgcn_readfirstlane(u - b * a.Nkv);
+    head = __builtin_amdgcn_readfirstlane(kvh * a.G + r - t * a.G);
+}
+__device__ __forceinline__ void pf_job(const FaArgs &a, int n_qt, int &qt, int &head, int &kvh, int &b, bool &second) {
     const uint32_t L = __builtin_amdgcn_workgroup_id_x();
     const uint32_t N = (uint32_t)(n_qt * a.Nh * a.B);
     const uint32_t nq = N / kXcds, nr = N % kXcds, x = L % kXcds, s0 = L / kXcds;
@@ -35,28 +44,21 @@ __device__ __forceinline__ void pf_job(const FaArgs &a, int n_qt, int &qt, int &
     const uint32_t cnt = min(kCusPerXcd, n_x - rnd * kCusPerXcd);
     const uint32_t s = (rnd & 1) ? rnd * kCusPerXcd + (cnt - 1 - w) : s0;
     const uint32_t J = x < nr ? x * (nq + 1) + s : nr * (nq + 1) + (x - nr) * nq + s;
-    const uint32_t per_u = (uint32_t)(a.G * n_qt);
-    const uint32_t u = J / per_u, r = J % per_u;
-    qt = __builtin_amdgcn_readfirstlane(n_qt - 1 - (int)(r / (uint32_t)a.G));
-    b = __builtin_amdgcn_readfirstlane((int)(u / (uint32_t)a.Nkv));
-    head = __builtin_amdgcn_readfirstlane((int)(u % (uint32_t)a.Nkv) * a.G + (int)(r % (uint32_t)a.G));
+    pf_place(a, n_qt, (int)J, qt, head, kvh, b);
     second = rnd == 1 && n_x >= 2 * kCusPerXcd;
 }
 
 // The same for a key-split grid of n_qt * Nh * B * a.pf_parts workgroups: the
 // parts of a job are neighbours on one XCD, jobs in pf_job's order.
-__device__ __forceinline__ void pf_unit(const FaArgs &a, int n_qt, int &job, int &part, int &qt, int &head, int &b) {
+__device__ __forceinline__ void pf_unit(const FaArgs &a, int n_qt, int &job, int &part, int &qt, int &head, int &kvh,
+                                        int &b) {
     const uint32_t L = __builtin_amdgcn_workgroup_id_x();
     const uint32_t N = (uint32_t)(n_qt * a.Nh * a.B) * (uint32_t)a.pf_parts;
     const uint32_t nq = N / kXcds, nr = N % kXcds, x = L % kXcds;
     const int U = (int)(x * nq + min(x, nr) + L / kXcds);
     job = __builtin_amdgcn_readfirstlane(div_fast(U, a.fd_parts));
     part = __builtin_amdgcn_readfirstlane(U - job * a.pf_parts);
-    const uint32_t per_u = (uint32_t)(a.G * n_qt), J = (uint32_t)job;
-    const uint32_t u = J / per_u, r = J % per_u;
-    qt = __builtin_amdgcn_readfirstlane(n_qt - 1 - (int)(r / (uint32_t)a.G));
-    b = __builtin_amdgcn_readfirstlane((int)(u / (uint32_t)a.Nkv));
-    head = __builtin_amdgcn_readfirstlane((int)(u % (uint32_t)a.Nkv) * a.G + (int)(r % (uint32_t)a.G));
+    pf_place(a, n_qt, job, qt, head, kvh, b);
 }
 
 // Tile classes of one (plane, query tile) row live in registers: lane l

@@ -52,17 +52,18 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
     // not fit this kernel's registers)
     static_assert(T == T_F16, "F16 K/V only");
 
+    warm_args();
     const int tid = (int)__builtin_amdgcn_workitem_id_x();
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n16 = lane & 15, g = lane >> 4;
-    int qt, head, b;
+    int qt, head, kvh, b;
     bool second = false;
-    pf_job(a, a.n_qt_w, qt, head, b, second);
+    pf_job(a, a.n_qt_w, qt, head, kvh, b, second);
     // (the staggered start of fa_mfma.hip: the CU's second workgroup of the
     // first pair waits ~2 us so that the two do not fetch in one burst)
     if (second) __builtin_amdgcn_s_sleep(64);
-    const int kvh = head / a.G, bk = b / a.rk3;
+    const int bk = div_fast(b, a.fd_rk3);
     const int q0w = qt * kPfWideBM + wave * 48;   // first query of this wave
     int qrow_c[3];                                // lane's query of block qb (rows past Sq: the last row)
 #pragma unroll
@@ -71,6 +72,7 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
     // Tile classes: the classifier labels 128-query tiles; this job's 192
     // rows lie within two of them (rows r0 .. r1), whose union class is
     // exact or conservative (mixed).
+    // (plain divisions: by multiplication they made the dense instance spill)
     const int plane = a.mask ? (b % a.m_ne3) * a.m_ne2 + head % a.m_ne2 : 0;
     const int r0 = qt * kPfWideBM / kPfBM;
     const int r1 = min((qt * kPfWideBM + kPfWideBM - 1) / kPfBM, (a.Sq - 1) / kPfBM);
@@ -125,8 +127,8 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
         sm_p0 = __builtin_amdgcn_readfirstlane(sm_p0);
         int len = a.Skv;
         if (a.sm_flags & kSmLengths) {
-            len = a.sm_len[b % a.sm_nlen];
-            if (a.sm_len_dev) len = sm_dev_load(a.sm_len_dev + b % a.sm_nlen);
+            len = a.sm_len[a.sm_nlen == 1 ? 0 : b];
+            if (a.sm_len_dev) len = sm_dev_load(a.sm_len_dev + (a.sm_nlen == 1 ? 0 : b));
             len = len < 0 ? 0 : len;
         }
         sm_hi = __builtin_amdgcn_readfirstlane(min(a.Skv, len));

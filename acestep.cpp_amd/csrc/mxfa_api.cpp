@@ -493,6 +493,7 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     a.M = a.Sq * a.G;
     a.fd_G = fast_div((uint32_t)a.G);
     a.fd_rk3 = fast_div((uint32_t)a.rk3);
+    a.fd_nkv = fast_div((uint32_t)a.Nkv);
     a.fd_m2 = fast_div((uint32_t)a.m_ne2);
     a.fd_m3 = fast_div((uint32_t)a.m_ne3);
     a.scale = p->scale;
@@ -605,6 +606,9 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         pl.wide = !split && !pl.narrow && kPfWide && k->type == MXFA_TYPE_F16 && a.softcap == 0.0f && !a.mask_unal &&
                   ((!mask && a.sm_flags == 0) || n_kt <= kPfWideMaskedMaxKt);
         a.n_qt_w = pl.wide ? (a.Sq + kPfWideBM - 1) / kPfWideBM : 0;
+        a.fd_unit = fast_div((uint32_t)(a.G * (pl.narrow ? a.n_qt_n : pl.wide ? a.n_qt_w : a.n_qt)));
+        a.fd_kt = fast_div((uint32_t)a.n_kt);
+        a.fd_qt = fast_div((uint32_t)a.n_qt);
         pl.n_planes = mask ? a.m_ne2 * a.m_ne3 : 0;
         pl.ws_bytes = mask ? (size_t)pl.n_planes * a.n_qt * a.n_kt_pad : 0;
         if (cls64_fit) {
@@ -710,7 +714,6 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     a.fd_rt = fast_div((uint32_t)a.row_tiles);
     a.fd_gy = fast_div((uint32_t)(a.Nkv * a.row_tiles));
     a.fd_hs = fast_div((uint32_t)std::max<int64_t>(1, n_splits / 2));
-    a.fd_nkv = fast_div((uint32_t)a.Nkv);
     a.fd_chunk = fast_div((uint32_t)chunk);
     // Paired splits (fa_decode.hip, make_tile): a dense grid of exactly two
     // workgroups per CU whose first half runs ahead of its second; the even

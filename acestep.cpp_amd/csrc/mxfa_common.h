@@ -71,7 +71,9 @@ struct FaArgs {
     int32_t m_ne2, m_ne3;
     int32_t Sq, Nh, B, Skv, Nkv, G, rk3;  // G = Nh/Nkv, rk3 = B/Bk
     FastDiv fd_G, fd_rk3, fd_m2, fd_m3;   // dividers of G, rk3, m_ne2, m_ne3
-    FastDiv fd_rt, fd_gy, fd_hs, fd_nkv, fd_chunk;   // decode: row_tiles, Nkv * row_tiles, n_splits / 2, Nkv, chunk
+    FastDiv fd_nkv;                       // Nkv
+    FastDiv fd_rt, fd_gy, fd_hs, fd_chunk;   // decode: row_tiles, Nkv * row_tiles, n_splits / 2, chunk
+    FastDiv fd_unit, fd_kt, fd_qt;        // prefill: G * query tiles of the kernel that runs, n_kt, n_qt
     int32_t M;                            // rows per (b, kv head) = Sq*G
     int32_t row_tiles;                    // decode kernel: ceil(M/16)
     float scale, softcap;                 // softcap == 0: off
@@ -107,7 +109,7 @@ struct FaArgs {
     int32_t sm_flags, sm_window, sm_pos0, sm_nlen;
     const int32_t *sm_len_dev;            // kSmDevice: lengths in device memory (else sm_len)
     const int32_t *sm_pos0_dev;           // kSmDevice: pos0 in device memory, or NULL (sm_pos0)
-    int32_t sm_len[kSmMaxLen];
+    int32_t sm_len[kSmMaxLen];            // (sm_nlen is 1 or B)
 };
 
 // Brings the kernel arguments (all but the structured mask's lengths) into
@@ -230,9 +232,9 @@ __host__ __device__ __forceinline__ void sm_row_range(const FaArgs &a, int b, in
     lo = 0;
     hi = a.Skv;
     if (a.sm_flags & kSmLengths) {
-        int len = a.sm_len[b % a.sm_nlen];
+        int len = a.sm_len[a.sm_nlen == 1 ? 0 : b];
 #if defined(__HIP_DEVICE_COMPILE__)
-        if (a.sm_len_dev) len = sm_dev_load(a.sm_len_dev + b % a.sm_nlen);
+        if (a.sm_len_dev) len = sm_dev_load(a.sm_len_dev + (a.sm_nlen == 1 ? 0 : b));
 #endif
         len = len < 0 ? 0 : len;
         hi = hi < len ? hi : len;
