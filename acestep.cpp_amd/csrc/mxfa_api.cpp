@@ -3,9 +3,12 @@
 // Validates ggml-style descriptors (the same contract ggml_flash_attn_ext
 // asserts), picks a kernel and launches it on the caller's stream:
 //   * split-KV decode kernel (fa_decode.hip) when few query rows share a
-//     KV head: decode (Sq = 1) and short prompts, and every Q8_0 K/V call;
-//   * MFMA prefill kernel (fa_mfma.hip) for long query runs (prefill, DiT),
-//     preceded by the mask tile classifier when a mask is given;
+//     KV head: decode (Sq = 1), short prompts, and what the prefill kernels
+//     do not take;
+//   * MFMA prefill kernels for long query runs (prefill, DiT, encoders) of
+//     32, 48 or 16 queries per wave (fa_mfma.hip, fa_wide.hip,
+//     fa_narrow.hip), preceded by the mask tile classifier when a mask is
+//     given and by the staging of Q8_0 K/V (q8_stage.hip);
 // and GGML_OP_SET_ROWS, the KV-cache write before each attention node
 // (set_rows.hip).
 // The only memory the engine owns is per (device, stream) and grow-only: a
@@ -575,20 +578,6 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         a.n_qt = (a.Sq + kPfBM - 1) / kPfBM;
         a.n_kt = (int32_t)n_kt;
         a.n_kt_pad = (a.n_kt + 3) & ~3;
-        // F16 calls without a mask (the DiT's self-attention: the reference
-        // casts K/V to F16 first) or with a dense mask over few key tiles
-        // (the DiT's cross-attention) take the kernel with 48 queries per
-        // wave: 192-query workgroups, each LDS operand read once for three
-        // MFMAs.  Same-box A/B against the 32-query kernel: C4 self 149.0
-        // against 164.0 us, C4 cross 35.1-35.6 against 37.5-37.6 us.  (BF16
-        // stays on the 32-query kernel: its P hi/lo pair does not fit the
-        // wide kernel's registers without spills.)
-        // The same rule holds for a dense mask and its structured form, so
-        // that the two stay on one kernel (bit-identical outputs).
-        // (mask rows without 8-byte alignment: the 32-query kernel, which
-        // reads the words of 0 / -inf tiles instead of their values)
-        // grids that 64-query workgroups fill better (the rule and its
-        // figures: fa_narrow.hip)
         // Few jobs over many key tiles: the tiles of a job dealt to several
         // workgroups (fa_mfma.hip, SPLIT), as many as fill the chip once, of
         // at least kPfSplitTiles tiles each.
@@ -603,8 +592,29 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         // figures: fa_narrow.hip)
         pl.narrow = !split && !q8 && (!mask || cls64_fit) && fa_narrow_serves(a);
         a.n_qt_n = pl.narrow ? (a.Sq + kPfNarrowBM - 1) / kPfNarrowBM : 0;
+        // F16 calls without a mask (the DiT's self-attention: the reference
+        // casts K/V to F16 first) or with a mask over few key tiles (the
+        // DiT's cross-attention) take the kernel with 48 queries per wave:
+        // 192-query workgroups, each LDS operand read once for three MFMAs.
+        // (BF16 stays on the 32-query kernel: its P hi/lo pair does not fit
+        // the wide kernel's registers without spills.)  Two workgroups of
+        // either kernel share a CU, so the grids decide for unmasked calls:
+        // they take it where it needs at most one workgroup per CU, or the
+        // 128-query grid more than two (in between its second round is
+        // nearly empty).  Measured, wide (128-query), 16 heads: 2 x 1250
+        // tokens 41.6 (43.6) us, 2 x 1500 48.8 (52.0), 2 x 1700 74.7 (60.4),
+        // 2 x 2000 88.7 (74.8), 2 x 2300 100.8 (114.4), 2 x 3000 144.5
+        // (157.2).  Masked calls keep it on every grid, which keeps a dense
+        // mask and its structured form bit-identical; that costs at most a
+        // few us (240 keys: 2 x 1085 24.0 (23.1), 2 x 2000 30.6 (26.3), 2 x
+        // 2300 30.8 (31.4), 2 x 3000 34.9 (37.6)).
+        // (mask rows without 8-byte alignment: the 32-query kernel, which
+        // reads the words of 0 / -inf tiles instead of their values)
+        const int64_t jobs_w = (int64_t)((a.Sq + kPfWideBM - 1) / kPfWideBM) * a.Nh * a.B;
+        const bool unmasked = !mask && a.sm_flags == 0;
+        const bool wide_grid = jobs > 2 * kDecCus || jobs_w <= kDecCus;
         pl.wide = !split && !pl.narrow && kPfWide && k->type == MXFA_TYPE_F16 && a.softcap == 0.0f && !a.mask_unal &&
-                  ((!mask && a.sm_flags == 0) || n_kt <= kPfWideMaskedMaxKt);
+                  (unmasked ? wide_grid : n_kt <= kPfWideMaskedMaxKt);
         a.n_qt_w = pl.wide ? (a.Sq + kPfWideBM - 1) / kPfWideBM : 0;
         a.fd_unit = fast_div((uint32_t)(a.G * (pl.narrow ? a.n_qt_n : pl.wide ? a.n_qt_w : a.n_qt)));
         a.fd_kt = fast_div((uint32_t)a.n_kt);
