@@ -317,6 +317,16 @@ __device__ __forceinline__ u16x8 bf16_lo8(f32x4 lo4, f32x4 hi4, u16x8 hi) {
     for (int i = 0; i < 8; i++) r[i] = bf16_lo(i < 4 ? lo4[i] : hi4[i - 4], hi[i]);
     return r;
 }
+// the same for f16 in the LDS decode kernel, which is bound by memory and
+// carries P to ~2^-22 so: its error does not depend on how the keys are split
+template <int T>
+__device__ __forceinline__ u16x8 p_lo8(f32x4 lo4, f32x4 hi4, u16x8 hi) {
+    if constexpr (T == T_BF16) return bf16_lo8(lo4, hi4, hi);
+    u16x8 r;
+#pragma unroll
+    for (int i = 0; i < 8; i++) r[i] = Mfma16<T_F16>::from_f32((i < 4 ? lo4[i] : hi4[i - 4]) - h2f_bits(hi[i]));
+    return r;
+}
 
 // Sum of 8 16-bit values of format T (the rounded probabilities that feed
 // the PV product) with v_dot2 against (1, 1): the softmax denominator then
