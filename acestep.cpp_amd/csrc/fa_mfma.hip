@@ -202,15 +202,6 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // dense masks' liveness words (class-3 tiles); the Q8_0 instance keeps
     // the mask reads (the host gives Q8_0 calls no words)
     constexpr bool kBits = !SM && !QQ8;
-    // growth of a row's maximum (exp2 domain) that raises its reference.  Odd
-    // mask rows raise it on any growth: a row's largest probability is then
-    // exactly 1 and rounds to itself, as far as the decode kernel, the path
-    // for them without this one, is from 64 bits.  Relative error, 8 -> 0:
-    // 1.9e-4 -> 1.7e-4 (2 x 1085 tokens under a window of 128, and over 238
-    // keys); the time, 28.9 -> 30.9 and 22.8 -> 24.1 us.  (Over the many keys
-    // of a split the one value does not count: 2.1e-4 both ways, 34.0 against
-    // 37.4 us on 333 tokens over 2133 keys.)
-    constexpr float kRaise = UNAL && !SPLIT ? 0.0f : 8.0f;
 
     // (work-item / group ids through the intrinsics: always inline, scalar)
     warm_args();
@@ -566,8 +557,12 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // probabilities of pair u (registers 2u, 2u+1) of a half, packed into
     // the P^T operand: k-slot 4u' + i <-> key 16kk + 8u' + 4h + i =
     // register 8kk + 4u' + i, i.e. operand kk holds registers 8kk..8kk+7.
-    // bf16: pl receives the lo parts (bf16_lo), which a second PV MFMA adds.
-    constexpr bool kLo = T == T_BF16;
+    // pl receives the lo parts (p_lo), which a second PV MFMA adds: bf16, and
+    // f16 under odd mask rows.  Without them such calls were further from 64
+    // bits than on the decode kernel, whose waves' own maxima round less (2 x
+    // 1085 tokens under a window of 128, or over 238 keys: 1.9e-4 against
+    // 1.7e-4; with them 2.4e-7, 28.9 -> 33.5 and 22.8 -> 25.4 us).
+    constexpr bool kLo = T == T_BF16 || UNAL;
     auto pair = [&](const f32x16 &sc, int u, float g, float mneg, u16x8 (&pw)[2], u16x8 (&pl)[2])
                     __attribute__((always_inline)) {
         const float p0 = fast_exp2(fmaf(sc[2 * u], g, mneg));
@@ -576,8 +571,8 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         pw[u >> 2][2 * (u & 3)] = h0;
         pw[u >> 2][2 * (u & 3) + 1] = h1;
         if constexpr (kLo) {
-            pl[u >> 2][2 * (u & 3)] = bf16_lo(p0, h0);
-            pl[u >> 2][2 * (u & 3) + 1] = bf16_lo(p1, h1);
+            pl[u >> 2][2 * (u & 3)] = p_lo<T>(p0, h0);
+            pl[u >> 2][2 * (u & 3) + 1] = p_lo<T>(p1, h1);
         }
     };
     // the denominator sums exactly the weights the PV product uses
@@ -670,7 +665,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
 
         // ---- R3: tile max, reference update (rare rescale) ----
         const float bmax = max_pair32(fmaxf(mxa, half_max(sb))) * g;
-        const bool any_need = __builtin_amdgcn_ballot_w64(bmax > m2 + kRaise) != 0;   // wave-uniform
+        const bool any_need = __builtin_amdgcn_ballot_w64(bmax > m2 + 8.0f) != 0;   // wave-uniform
         if (any_need) {
             const float mnew = fmaxf(m2, bmax);
             const float alpha = (m2 == -INFINITY) ? 1.0f : fast_exp2(m2 - mnew);

@@ -30,7 +30,7 @@
 // (the layout of fa_wide.hip), so a query's scores are spread over lanes n,
 // n+16, n+32, n+48; the reference max is equal across them, and the row
 // maximum over the four lanes is taken only when some lane's own maximum
-// exceeds the reference.
+// exceeds the reference by more than 8 (exp2 domain).
 
 #include "fa_prefill.h"
 #include "once_per_device.h"
@@ -46,11 +46,7 @@ template <int NST> constexpr int narrow_lds() { return NST * kNarrowStage; }
 template <int T, int MODE, bool CAP, int NST>
 __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
     constexpr bool SM = MODE == kNarrowSm, DENSE = MODE == kNarrowDense || MODE == kNarrowUnal;
-    constexpr bool kLo = T == T_BF16;       // P as a hi/lo pair (bf16_lo)
-    // as fa_mfma.hip under odd mask rows, in every mode, which keeps the forms
-    // of one mask bit-identical: eight encoder layers of 437 tokens 1.9e-4 ->
-    // 1.7e-4 from 64 bits, 92.6 -> 97.9 us
-    constexpr float kRaise = 0.0f;
+    constexpr bool kLo = T == T_BF16 || MODE == kNarrowUnal;   // P as a hi/lo pair (fa_mfma.hip)
     constexpr int kPer = 8 + (DENSE ? 1 : 0);   // copies per stage
     using MF = Mfma16<T>;
     using V8 = typename MF::v8;
@@ -264,7 +260,7 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
             const float p = fast_exp2(fmaf(s[kb][i], gs, mneg));
             const uint16_t h = MF::from_f32(p);
             pw[4 * kb + i] = h;
-            if constexpr (kLo) pl[4 * kb + i] = bf16_lo(p, h);
+            if constexpr (kLo) pl[4 * kb + i] = p_lo<T>(p, h);
         }
     };
     auto psum = [&](const u16x8 &pw, const u16x8 &pl) __attribute__((always_inline)) -> float {
@@ -355,7 +351,7 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
 
         // ---- R3: tile max, reference update (rare) ----
         const float bmax = fmaxf(mxa, max8(sb)) * gs;
-        if (__builtin_amdgcn_ballot_w64(bmax > m2 + kRaise) != 0) {   // wave-uniform
+        if (__builtin_amdgcn_ballot_w64(bmax > m2 + 8.0f) != 0) {   // wave-uniform
             const float rmax = max_pair16(max_half32(bmax));         // over the query's four lanes
             const float mnew = fmaxf(m2, rmax);
             const float alpha = (m2 == -INFINITY) ? 1.0f : fast_exp2(m2 - mnew);

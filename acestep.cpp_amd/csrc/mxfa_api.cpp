@@ -531,7 +531,7 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     // DiT's and the encoders' [S, S] masks for 3 of 4 lengths S.  Measured
     // per call against the scalar decode kernel, which streams all of K and
     // V for every 16 query rows: 2 x 1085 tokens at 16 / 8 heads under a
-    // window of 128, 29.2 against 123.7 us; over 238 encoder keys, 22.3
+    // window of 128, 33.7 against 123.7 us; over 238 encoder keys, 25.4
     // against 70.7 us; eight layers of 437 tokens, four of them under a
     // window, 146.9 against 262.7 us.
     if (mask) {

@@ -317,8 +317,14 @@ __device__ __forceinline__ u16x8 bf16_lo8(f32x4 lo4, f32x4 hi4, u16x8 hi) {
     for (int i = 0; i < 8; i++) r[i] = bf16_lo(i < 4 ? lo4[i] : hi4[i - 4], hi[i]);
     return r;
 }
-// the same for f16 in the LDS decode kernel, which is bound by memory and
-// carries P to ~2^-22 so: its error does not depend on how the keys are split
+// the same for f16, which carries P to ~2^-22 so: the LDS decode kernel (its
+// error then does not depend on how the keys are split) and the prefill
+// kernels under odd mask rows
+template <int T>
+__device__ __forceinline__ uint16_t p_lo(float p, uint16_t h) {
+    if constexpr (T == T_BF16) return bf16_lo(p, h);
+    else return Mfma16<T_F16>::from_f32(p - h2f_bits(h));
+}
 template <int T>
 __device__ __forceinline__ u16x8 p_lo8(f32x4 lo4, f32x4 hi4, u16x8 hi) {
     if constexpr (T == T_BF16) return bf16_lo8(lo4, hi4, hi);

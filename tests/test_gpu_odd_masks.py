@@ -62,12 +62,14 @@ def test_odd_mask_rows(mx, Sq, Skv, mask, kw, extra, shift):  # noqa: F811
 
 
 def test_odd_rows_equal_padded_rows(mx):  # noqa: F811
-    """The same mask in odd rows and in rows padded to 8 bytes: bit for bit."""
+    """The same mask in odd rows (P as a hi/lo pair) and in rows padded to 8
+    bytes (weights off by at most 2^-11 of themselves: 2 * 2^-11 * max|V|)."""
     c = _rand_case(751, B=2, Sq=261, Nh=8, Nkv=2, Skv=337, mask="random")
     odd = run_gpu(mx, c)
     c.mask = _repitch(c.mask, 3, 0)
     c.mask.ne = (340,) + tuple(c.mask.ne[1:])   # rows of 340 entries, 8-byte aligned
-    assert np.array_equal(odd, run_gpu(mx, c))
+    bound = 2.1 * 2.0 ** -11 * np.abs(c.v.buf.view(np.float16)).max()
+    assert np.abs(odd - run_gpu(mx, c)).max() <= bound
 
 
 def test_odd_rows_under_capture_without_reserve(mx):  # noqa: F811

@@ -44,7 +44,11 @@ def test_split_structured_equals_dense(mx, spec, Skv):  # noqa: F811
     q, k, v = (mx.upload(t) for t in (c.q, c.k, c.v))
     out = mx.flash_attn_ext_masked(q, k, v, mx.mask_spec(**spec), c.scale)
     torch.cuda.synchronize()
-    assert np.array_equal(mx.output_tensor(out).cpu().numpy(), dense)
+    got = mx.output_tensor(out).cpu().numpy()
+    if Skv % 4:   # odd mask rows carry P as a hi/lo pair; the spec's weights are off by at most 2^-11 of themselves
+        assert np.abs(got - dense).max() <= 2.1 * 2.0 ** -11 * np.abs(c.v.buf.view(np.float16)).max()
+    else:
+        assert np.array_equal(got, dense)
 
 
 def test_split_fully_masked_rows(mx):  # noqa: F811
