@@ -178,6 +178,14 @@ __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint
     }
 }
 
+// The 12 wait states between an MFMA of 8 passes and a vector read of its
+// result, where a branch lies between the two: there the compiler's own count
+// has come out short (some reads after 4).  BF16 prefills under an aligned
+// mask of 3 or 4 key tiles then took a stale score for 2 keys of every other
+// tile (3.5e-2 off) once the branch target was in the instruction cache.
+// tests/test_mfma_wait_states.py counts them in the built code.
+__device__ __forceinline__ void mfma_done(f32x16 &x) { asm volatile("s_nop 7\n\ts_nop 3" : "+v"(x)); }
+
 // CAP: logit softcap on (a per-call constant; its tanh path is compiled only
 // into the instances that need it, so it costs the common path no registers).
 // SM: structured mask (a.sm_*): tile classes and per-element liveness are
@@ -639,7 +647,10 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
             if (do_issue) copy(t);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (general) general_x(sa, key0, cl, (uint32_t)tbits);
+        if (general) {
+            mfma_done(sa);
+            general_x(sa, key0, cl, (uint32_t)tbits);
+        }
         __builtin_amdgcn_sched_barrier(0);
 
         // ---- R2: QK b | softmax a (speculative) ----
@@ -650,8 +661,13 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         for (int t = 0; t < 8; t++) {
             fetch(8 + t + kPfLook);
             sb = MF::run(__builtin_bit_cast(V8, op[(8 + t) & 7]), qb[t], t == 0 ? f32x16{} : sb);
-            if (t == 0) mxa = half_max(sa);
-            else pair(sa, t - 1, g, mneg0, pa, pal);
+            if (t == 0) {   // (waited for behind the MFMA, which takes as long)
+                __builtin_amdgcn_sched_barrier(0);
+                mfma_done(sa);
+                mxa = half_max(sa);
+            } else {
+                pair(sa, t - 1, g, mneg0, pa, pal);
+            }
             if (t == 7) pair(sa, 7, g, mneg0, pa, pal);
             __builtin_amdgcn_sched_barrier(0);
         }
