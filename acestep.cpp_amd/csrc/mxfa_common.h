@@ -401,14 +401,16 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // buffer.  Compiler-generated waits for other vector loads stay correct: a
 // copy unknown to the compiler only makes them wait longer (counters retire
 // in order).
+// The s_nop is the wait state that a scalar write of M0 needs ahead of an LDS
+// copy (the compiler keeps it for its own copies, not inside inline assembly).
 __device__ __forceinline__ void dma16_at(const void *g, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(g)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(g)
                  : "memory", "m0");
 }
 // The same with 4 bytes per lane (4-byte aligned source): lane l's bytes
 // land at lds_addr + 4*l.
 __device__ __forceinline__ void dma4_at(const void *g, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" : : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(g)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(g)
                  : "memory", "m0");
 }
 
@@ -430,7 +432,7 @@ __device__ __forceinline__ i32x4 buf_rsrc(const void *base, uint32_t bytes) {
 // lds_addr + 16*l.  Same wait contract as dma16 (callers wait with
 // MXFA_WAIT_VMCNT before reading the buffer).
 __device__ __forceinline__ void dma16_buf(const i32x4 &rsrc, uint32_t voff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                  :
                  : "s"(lds_addr), "v"(voff), "s"(rsrc)
                  : "memory", "m0");
@@ -438,7 +440,7 @@ __device__ __forceinline__ void dma16_buf(const i32x4 &rsrc, uint32_t voff, uint
 
 // The same with 4 bytes per lane (bytes land at lds_addr + 4*l).
 __device__ __forceinline__ void dma4_buf(const i32x4 &rsrc, uint32_t voff, uint32_t lds_addr) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
                  :
                  : "s"(lds_addr), "v"(voff), "s"(rsrc)
                  : "memory", "m0");
