@@ -140,8 +140,25 @@ __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint
             live |= (uint32_t)(k + i < a.Skv && !ninf) << (4 * pass + i);
         }
     }
-    // wave votes (3 bits per half), then one barrier across the 4 waves
+    // wave votes (3 bits per half), then one barrier across the 4 waves; with
+    // them go the keys live for some of the wave's rows (lo and hi word per
+    // half: the 8 lanes of a word, then the wave's 4 rows of a pass)
     __shared__ uint32_t votes[4];
+    __shared__ __attribute__((aligned(16))) uint32_t seen[4][4];
+#pragma unroll
+    for (int hf = 0; hf < 2; hf++) {
+        uint32_t n = live >> (16 * hf) & 0xFFFFu;
+        n |= n >> 8;
+        n = ((n | n >> 4) & 0xFu) << (4 * (c4 & 7));
+        n |= dpp_u32<0xB1>(n);
+        n |= dpp_u32<0x4E>(n);
+        n |= dpp_u32<0x141>(n);
+        const auto r16 = __builtin_amdgcn_permlane16_swap(n, n, false, false);
+        n = r16[0] | r16[1];
+        const auto r32 = __builtin_amdgcn_permlane32_swap(n, n, false, false);
+        n = r32[0] | r32[1];
+        if ((threadIdx.x & 0x37) == 0) seen[threadIdx.x >> 6][2 * hf + (c4 >> 3)] = n;   // lanes 0 and 8
+    }
     uint32_t vote = 0;
 #pragma unroll
     for (int hf = 0; hf < 2; hf++) {
@@ -155,7 +172,23 @@ __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint
     auto class_of = [&](uint32_t any) -> int {
         return !(any & 1u) ? 0 : (!(any & 2u) ? 1 : (!(any & 4u) && a.tile_bits ? 3 : 2));
     };
-    const int c = class_of((any2 | any2 >> 4) & 7u), c0 = class_of(any2 & 7u), c1 = class_of(any2 >> 4);
+    int c = class_of((any2 | any2 >> 4) & 7u), c0 = class_of(any2 & 7u), c1 = class_of(any2 >> 4);
+    if (a.tile_keys && c >= 2) {   // (uniform) the keys live for some row of each half
+        uint64_t h[2];
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++) {
+            u32x2 w = {0u, 0u};
+#pragma unroll
+            for (int i = 0; i < 4; i++) w |= *(const u32x2 *)&seen[i][2 * hf];
+            h[hf] = __builtin_bit_cast(uint64_t, w);
+        }
+        const uint64_t all = ~0ull >> (64 - min(a.Skv - k_lo, kPfBN));   // (keys past Skv are no one's)
+        if ((h[0] | h[1]) != all) c |= kTileDeadKeys;
+        if (c0 >= 2 && h[0] != all) c0 |= kTileDeadKeys;
+        if (c1 >= 2 && h[1] != all) c1 |= kTileDeadKeys;
+        if (threadIdx.x < 2)
+            a.tile_keys[((int64_t)plane * 2 * a.n_qt + 2 * qt + threadIdx.x) * a.n_kt + kt] = threadIdx.x ? h[1] : h[0];
+    }
     if (threadIdx.x == 0) {
         cls[((int64_t)plane * a.n_qt + qt) * a.n_kt_pad + kt] = (uint8_t)c;
         if (cls64) {
@@ -164,7 +197,7 @@ __global__ void __launch_bounds__(256) mask_classify_kernel(const FaArgs a, uint
             p[a.n_kt_pad] = (uint8_t)c1;
         }
     }
-    if (c == 3 || (cls64 && (c0 == 3 || c1 == 3))) {   // (uniform) the liveness words of the tile's rows
+    if ((c & 3) == 3 || (cls64 && ((c0 & 3) == 3 || (c1 & 3) == 3))) {   // (uniform) the liveness words of the tile's rows
         uint64_t *bits = a.tile_bits + (((int64_t)plane * a.n_qt + qt) * a.n_kt + kt) * kPfBM;
 #pragma unroll
         for (int pass = 0; pass < kPfBM / 16; pass++) {
@@ -245,6 +278,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // there needs no per-element test (class 1); the others test each key
     // against the lane's own row range [row_lo, row_hi).
     int sm_kt_first = 0, sm_kt_end = 0, sm_in_lo = 0, sm_in_hi = 0, row_lo = 0, row_hi = 0;
+    int sm_lo = 0, sm_hi = 0, sm_kt_lo = -1, sm_kt_hi = -1;   // the keys the rows see together, their ragged end tiles
     if constexpr (SM) {
         const int q_first = qt * kPfBM, q_last = min(q_first + kPfBM, a.Sq) - 1;
         int lo_f, hi_f, lo_l, hi_l;
@@ -252,6 +286,10 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         sm_row_range(a, b, q_last, lo_l, hi_l);
         sm_kt_first = __builtin_amdgcn_readfirstlane(max(lo_f, 0) / kPfBN);
         sm_kt_end = __builtin_amdgcn_readfirstlane(lo_f < hi_l ? (hi_l + kPfBN - 1) / kPfBN : 0);
+        sm_lo = __builtin_amdgcn_readfirstlane(lo_f);
+        sm_hi = __builtin_amdgcn_readfirstlane(hi_l);
+        if (sm_lo % kPfBN) sm_kt_lo = sm_kt_first;
+        if (sm_hi % kPfBN) sm_kt_hi = sm_kt_end - 1;
         sm_in_lo = __builtin_amdgcn_readfirstlane(lo_l);
         sm_in_hi = __builtin_amdgcn_readfirstlane(hi_f);
         sm_row_range(a, b, qrow_c, row_lo, row_hi);
@@ -274,7 +312,9 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         }
     };
     auto class_of = [&](int kt) __attribute__((always_inline)) -> int {
-        if constexpr (SM) return (kt * kPfBN >= sm_in_lo && kt * kPfBN + kPfBN <= sm_in_hi) ? 1 : 2;
+        if constexpr (SM)
+            return (kt * kPfBN >= sm_in_lo && kt * kPfBN + kPfBN <= sm_in_hi) ? 1
+                   : kt == sm_kt_lo || kt == sm_kt_hi ? 2 | kTileDeadKeys : 2;
         else return tc.at(kt);
     };
     // this workgroup's tiles: every parts-th live one from the part-th
@@ -459,6 +499,9 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
         }
     }
 
+    WaveKeys wk;   // (lands with Q)
+    if (tc.present) wk.init(a, plane, 2 * qt, 2, wave, lane);
+
     // LDS operand addresses.  QK: K operand of dim-step t for key l32 of a
     // half: chunk (2t + h) ^ swz_k(l32) of row l32.  PV: V^T operand of dim
     // tile dt for the 16-key step kk (keys 16kk + 8u + tr_key of a half):
@@ -613,7 +656,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // stage NST go out one per QK MFMA of half a (SPREAD): spread so, their
     // issue (~40 cycles each, with the LDS address set per copy) hides under
     // the matrix cores instead of holding up the tile's first MFMAs.
-    auto tile = [&](auto st_c, int kt, auto nst_c, int kn, uint64_t tbits) __attribute__((always_inline)) {
+    auto tile = [&](auto st_c, int kt, auto nst_c, int kn, int cls, uint64_t tbits) __attribute__((always_inline)) {
         constexpr int NST = decltype(nst_c)::value;
         const bool do_issue = SPREAD && kn < n_kt;   // uniform
         const uint32_t nl0 = lds0 + NST * kStageBytes + (uint32_t)(16 * wave) * 256u;
@@ -622,7 +665,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
             if (c & 1) dma16_buf(rv, vv[c >> 1] + nvo, nl0 + kTileBytes + 4 * (c >> 1) * 256);
             else dma16_buf(rk, vk[c >> 1] + nko, nl0 + 4 * (c >> 1) * 256);
         };
-        const int cl = __builtin_amdgcn_readfirstlane(class_of(kt));
+        const int cl = cls & 3;
         const int key0 = kt * kPfBN;
         const bool general =
             __builtin_amdgcn_readfirstlane((int)(cl >= 2 || key0 + kPfBN > a.Skv || !lean_ok)) != 0;
@@ -740,34 +783,50 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     const uint64_t *brow = (kBits && tc.present && a.tile_bits)
                                ? a.tile_bits + ((int64_t)plane * a.n_qt + qt) * a.n_kt * kPfBM + wave * 32 + l32
                                : nullptr;
-    auto load_bits = [&](int k) __attribute__((always_inline)) -> uint64_t {
-        if (!kBits || brow == nullptr || k >= n_kt || __builtin_amdgcn_readfirstlane(class_of(k)) != 3) return 0;
+    auto load_bits = [&](int k, int cls) __attribute__((always_inline)) -> uint64_t {
+        if (!kBits || brow == nullptr || (cls & 3) != 3) return 0;
         return brow[(int64_t)k * kPfBM];
+    };
+    // V of keys that no row of the job sees, in stage ST (fa_prefill.h)
+    auto drop_dead = [&](int kt, int cls, int st) __attribute__((always_inline)) {
+        if (__builtin_expect(!(cls & kTileDeadKeys), 1)) return;
+        const uint32_t dead = SM ? dead_outside(sm_lo, sm_hi, kt * kPfBN + 16 * wave) : wk.dead(kt, wave, lane);
+        zero_dead_v(dead, lds0 + (uint32_t)(st * kStageBytes + kTileBytes + 16 * wave * 256));
     };
     std::integral_constant<int, 0> st0;
     std::integral_constant<int, 1> st1;
     int ofree = 1;   // the stage no tile still reads at the end
-    uint64_t cbits = load_bits(kt);
+    // (a tile's class is looked up once, a tile ahead; past the last: 0)
+    auto tile_class = [&](int k) __attribute__((always_inline)) -> int {
+        return k < n_kt ? __builtin_amdgcn_readfirstlane(class_of(k)) : 0;
+    };
+    int cls = tile_class(kt);
+    uint64_t cbits = load_bits(kt, cls);
     while (kt < n_kt) {
-        int kn = after(kt);
+        int kn = after(kt), ncls = tile_class(kn);
         MXFA_WAIT_VMCNT(0);
+        drop_dead(kt, cls, 0);
         __builtin_amdgcn_s_barrier();
         if (!SPREAD && kn < n_kt) issue(kn, st1);
-        uint64_t nbits = load_bits(kn);
-        tile(st0, kt, st1, kn, cbits);
+        uint64_t nbits = load_bits(kn, ncls);
+        tile(st0, kt, st1, kn, cls, cbits);
         cbits = nbits;
         ofree = 1;
         kt = kn;
+        cls = ncls;
         if (kt >= n_kt) break;
         kn = after(kt);
+        ncls = tile_class(kn);
         MXFA_WAIT_VMCNT(0);
+        drop_dead(kt, cls, 1);
         __builtin_amdgcn_s_barrier();
         if (!SPREAD && kn < n_kt) issue(kn, st0);
-        nbits = load_bits(kn);
-        tile(st1, kt, st0, kn, cbits);
+        nbits = load_bits(kn, ncls);
+        tile(st1, kt, st0, kn, cls, cbits);
         cbits = nbits;
         ofree = 0;
         kt = kn;
+        cls = ncls;
     }
 
     lsum = sum_pair32(lsum);

@@ -74,6 +74,7 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
     }
     // structured mask: as fa_mfma.hip, over the job's 64 rows
     int sm_kt_first = 0, sm_kt_end = 0, sm_in_lo = 0, sm_in_hi = 0, row_lo = 0, row_hi = 0;
+    int sm_lo = 0, sm_hi = 0, sm_kt_lo = -1, sm_kt_hi = -1;   // the keys the rows see together, their ragged end tiles
     if constexpr (SM) {
         const int q_first = qt * kPfNarrowBM, q_last = min(q_first + kPfNarrowBM, a.Sq) - 1;
         int lo_f, hi_f, lo_l, hi_l;
@@ -81,6 +82,10 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
         sm_row_range(a, b, q_last, lo_l, hi_l);
         sm_kt_first = __builtin_amdgcn_readfirstlane(max(lo_f, 0) / kPfBN);
         sm_kt_end = __builtin_amdgcn_readfirstlane(lo_f < hi_l ? (hi_l + kPfBN - 1) / kPfBN : 0);
+        sm_lo = __builtin_amdgcn_readfirstlane(lo_f);
+        sm_hi = __builtin_amdgcn_readfirstlane(hi_l);
+        if (sm_lo % kPfBN) sm_kt_lo = sm_kt_first;
+        if (sm_hi % kPfBN) sm_kt_hi = sm_kt_end - 1;
         sm_in_lo = __builtin_amdgcn_readfirstlane(lo_l);
         sm_in_hi = __builtin_amdgcn_readfirstlane(hi_f);
         sm_row_range(a, b, qrow, row_lo, row_hi);
@@ -95,7 +100,9 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
         }
     };
     auto class_of = [&](int kt) __attribute__((always_inline)) -> int {
-        if constexpr (SM) return (kt * kPfBN >= sm_in_lo && kt * kPfBN + kPfBN <= sm_in_hi) ? 1 : 2;
+        if constexpr (SM)
+            return (kt * kPfBN >= sm_in_lo && kt * kPfBN + kPfBN <= sm_in_hi) ? 1
+                   : kt == sm_kt_lo || kt == sm_kt_hi ? 2 | kTileDeadKeys : 2;
         else return tc.at(kt);
     };
     const char *mplane = DENSE ? a.mask + (int64_t)(mod_fast(head, a.fd_m2, a.m_ne2)) * a.m_nb2 + (int64_t)mod_fast(b, a.fd_m3, a.m_ne3) * a.m_nb3 : a.q;
@@ -179,6 +186,9 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
             for (int t = 0; t < 4; t++) qv[t] = __builtin_bit_cast(V8, cvt8<T>(x[t][0], x[t][1]));
         }
     }
+
+    WaveKeys wk;   // (lands with Q)
+    if constexpr (DENSE) wk.init(a, plane, qt, 1, wave, lane);
 
     // (Q is waited for here: the wait the compiler would otherwise put at the
     // operands' first use, inside the tile loop, drains the copies in flight)
@@ -277,10 +287,10 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
     // copies of tile kn (kn < n_kt) into stage sn go out one per two steps
     // of R1 and R2.
     constexpr int kLook = 6, kRing = 8;
-    auto tile = [&](int kt, int st, int kn, int sn) __attribute__((always_inline)) {
+    auto tile = [&](int kt, int cls, int st, int kn, int sn) __attribute__((always_inline)) {
         const bool do_issue = kn < n_kt;   // uniform
         if (do_issue) words(kn, sn);
-        const int cl = __builtin_amdgcn_readfirstlane(class_of(kt));
+        const int cl = cls & 3;
         const int key0 = kt * kPfBN;
         const bool general =
             __builtin_amdgcn_readfirstlane((int)(cl >= 2 || key0 + kPfBN > a.Skv || !lean_ok)) != 0;
@@ -394,6 +404,7 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
     // every wave is done with the stage the next copies go to), compute.
     int st = 0;
     while (kq[0] < n_kt) {
+        const int cls = __builtin_amdgcn_readfirstlane(class_of(kq[0]));
         if constexpr (NST == 4) {
             if (kq[2] < n_kt) MXFA_WAIT_VMCNT(2 * kPer);
             else if (kq[1] < n_kt) MXFA_WAIT_VMCNT(kPer);
@@ -402,8 +413,14 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
             static_assert(NST == 2, "stages");
             MXFA_WAIT_VMCNT(0);
         }
+        if constexpr (MODE != kNarrowNone)   // V of keys that no row of the job sees (fa_prefill.h)
+            if (__builtin_expect(cls & kTileDeadKeys, 0)) {
+                const uint32_t dead =
+                    SM ? dead_outside(sm_lo, sm_hi, kq[0] * kPfBN + 16 * wave) : wk.dead(kq[0], wave, lane);
+                zero_dead_v(dead, lds0 + (uint32_t)(st * kNarrowStage + kTileBytes + 16 * wave * 256));
+            }
         __builtin_amdgcn_s_barrier();
-        tile(kq[0], st, kq[NST - 1], st == 0 ? NST - 1 : st - 1);
+        tile(kq[0], cls, st, kq[NST - 1], st == 0 ? NST - 1 : st - 1);
 #pragma unroll
         for (int i = 0; i < NST - 1; i++) kq[i] = kq[i + 1];
         kq[NST - 1] = next_live(kq[NST - 2] + 1);

@@ -95,12 +95,12 @@ struct TileClasses {
 
 // Class bytes (0 all -inf, 1 all zero, 2 mixed) of the union of two row
 // ranges' tiles, four at a time: equal classes stand, different ones make
-// the tile mixed.
+// the tile mixed, with dead keys to look for.
 __device__ __forceinline__ uint32_t class_union4(uint32_t x, uint32_t y) {
     const uint32_t d = x ^ y;
     const uint32_t nz = (((d & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | d) & 0x80808080u;   // bit 7: byte differs
     const uint32_t m = (nz >> 7) * 0xFFu;
-    return (x & ~m) | (0x02020202u & m);
+    return (x & ~m) | (0x01010101u * (2 | kTileDeadKeys) & m);
 }
 
 // Max of a lane's value and the same register of lane l ^ 32 (one
@@ -109,5 +109,65 @@ __device__ __forceinline__ float max_pair32(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x),
                                                     false, false);
     return fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+}
+
+// Keys that no query of a workgroup may see have P = 0, but 0 times a NaN or
+// an infinity in a masked V slot would be NaN in every row of the tile (ggml
+// skips such keys: ggml-cpu/ops.cpp, flash_attn_ext_f16_one_chunk).  Each wave
+// zeroes the V rows of such keys among the 16 it has copied, before the
+// tile's barrier, in the tiles that have any (kTileDeadKeys).  The other tiles
+// pay a test: 2 x 1085 tokens under a window of 128 34.1 -> 34.4 us, over 238
+// encoder keys with 31 of padding 25.7 -> 26.2, eight encoder layers 96.6 ->
+// 97.9.  (Measured and dropped: masking the V operands of mixed tiles, 5 to 8
+// % on the DiT's masked calls; leaving the rows out of the copies, 3 %; a look
+// at O and a second pass where it is not finite, 2 %, and 10 % where that pass
+// made the compiler spill.)
+//
+// WaveKeys: the keys that some row of the job may see among the 16 of each
+// tile that this wave copies; lane l holds those of tile base + l.
+struct WaveKeys {
+    const uint32_t *p = nullptr;   // this wave's half word of tile 0, first row (NULL: not known)
+    int rows = 0, n_kt = 0, base = 0;
+    uint32_t u = 0;
+    __device__ __forceinline__ void load(int base_, int lane) {
+        base = base_;
+        u = 0;
+        if (base + lane < n_kt)
+            for (int r = 0; r < rows; r++) u |= p[2 * ((int64_t)r * n_kt + base + lane)];
+    }
+    // row0: the job's first 64-query row of the plane (of 2 * a.n_qt)
+    __device__ __forceinline__ void init(const FaArgs &a, int plane, int row0, int rows_, int wave, int lane) {
+        if (!a.tile_keys) return;
+        rows = min(rows_, 2 * a.n_qt - row0);
+        n_kt = a.n_kt;
+        p = (const uint32_t *)(a.tile_keys + ((int64_t)plane * 2 * a.n_qt + row0) * n_kt) + (wave >> 1);
+        load(0, lane);
+    }
+    // bit j: no query sees key 16 wave + j of tile kt (uniform; every lane active)
+    __device__ __forceinline__ uint32_t dead(int kt, int wave, int lane) {
+        if (!p) return 0;
+        if (kt - base >= 64 || kt < base) load(kt & ~63, lane);
+        return ~((uint32_t)__builtin_amdgcn_readlane(u, kt & 63) >> (16 * (wave & 1))) & 0xFFFFu;
+    }
+};
+// The same where the rows together see the keys [lo, hi); key0: the wave's first.
+__device__ __forceinline__ uint32_t dead_outside(int lo, int hi, int key0) {
+    const int l = min(max(lo - key0, 0), 16), h = min(max(hi - key0, 0), 16);
+    return ~((0xFFFFu << l) & ((1u << h) - 1u)) & 0xFFFFu;
+}
+// v: LDS address of the wave's first V row (copy c: key 4c + lane / 16, 16
+// bytes a lane).  Three registers: the lane id is counted anew and the zeros
+// go out as dwords, or fa_wide.hip, which has none to spare, spills.
+__device__ __forceinline__ void zero_dead_v(uint32_t dead, uint32_t v) {
+    const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const uint32_t addr = v + 16 * lane;
+    for (uint32_t c = 0; c < 4; c++)
+        if ((dead >> (4 * c + (lane >> 4))) & 1u)
+            asm volatile("ds_write_b32 %0, %1\n\tds_write_b32 %0, %1 offset:4\n\t"
+                         "ds_write_b32 %0, %1 offset:8\n\tds_write_b32 %0, %1 offset:12"
+                         :
+                         : "v"(addr + 1024 * c), "v"(0u)
+                         : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 }  // namespace mxfa

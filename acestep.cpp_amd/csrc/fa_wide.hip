@@ -77,11 +77,16 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
     const int r0 = qt * kPfWideBM / kPfBM;
     const int r1 = min((qt * kPfWideBM + kPfWideBM - 1) / kPfBM, (a.Sq - 1) / kPfBM);
     TileClasses tc{0u, 0u, MASKED && a.tile_class != nullptr};
+    uint32_t cls0 = 0, cls1 = 0;   // the class bytes of rows r0, r1
     if (tc.present) {
         const uint32_t *row0 = (const uint32_t *)(a.tile_class + ((int64_t)plane * a.n_qt + r0) * a.n_kt_pad);
         const uint32_t *row1 = (const uint32_t *)(a.tile_class + ((int64_t)plane * a.n_qt + r1) * a.n_kt_pad);
         const int lane4 = 4 * lane;
-        if (lane4 < a.n_kt) tc.w0 = class_union4(row0[lane], row1[lane]);
+        if (lane4 < a.n_kt) {
+            cls0 = row0[lane];
+            cls1 = row1[lane];
+            tc.w0 = class_union4(cls0, cls1);
+        }
         if (256 + lane4 < a.n_kt) tc.w1 = class_union4(row0[64 + lane], row1[64 + lane]);
     }
     // Mask rows of this (batch, head) plane through a buffer resource (as
@@ -107,6 +112,7 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
     // [lo(first), hi(last)) are skipped, tiles inside [lo(last), hi(first))
     // need no per-element test.
     int sm_p0 = 0, sm_hi = a.Skv, sm_kt_first = 0, sm_kt_end = 0, sm_in_lo = 0, sm_in_hi = 0;
+    int sm_lo = 0, sm_key_end = 0, sm_kt_lo = -1, sm_kt_hi = -1;   // the keys the rows see together, their ragged end tiles
     auto row_range = [&](int q, int &lo, int &hi) __attribute__((always_inline)) {
         const int p = sm_p0 + q;
         lo = 0;
@@ -138,6 +144,10 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
         row_range(q_last, lo_l, hi_l);
         sm_kt_first = __builtin_amdgcn_readfirstlane(max(lo_f, 0) / kPfBN);
         sm_kt_end = __builtin_amdgcn_readfirstlane(lo_f < hi_l ? (hi_l + kPfBN - 1) / kPfBN : 0);
+        sm_lo = __builtin_amdgcn_readfirstlane(lo_f);
+        sm_key_end = __builtin_amdgcn_readfirstlane(hi_l);
+        if (sm_lo % kPfBN) sm_kt_lo = sm_kt_first;
+        if (sm_key_end % kPfBN) sm_kt_hi = sm_kt_end - 1;
         sm_in_lo = __builtin_amdgcn_readfirstlane(lo_l);
         sm_in_hi = __builtin_amdgcn_readfirstlane(hi_f);
     }
@@ -183,7 +193,9 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
         }
     };
     auto class_of = [&](int kt) __attribute__((always_inline)) -> int {
-        if constexpr (SM) return (kt * kPfBN >= sm_in_lo && kt * kPfBN + kPfBN <= sm_in_hi) ? 1 : 2;
+        if constexpr (SM)
+            return (kt * kPfBN >= sm_in_lo && kt * kPfBN + kPfBN <= sm_in_hi) ? 1
+                   : kt == sm_kt_lo || kt == sm_kt_hi ? 2 | kTileDeadKeys : 2;
         else return tc.at(kt);
     };
 
@@ -229,6 +241,27 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
         for (int qb = 0; qb < 3; qb++)
 #pragma unroll
             for (int t = 0; t < 4; t++) qv[qb][t] = __builtin_bit_cast(V8, cvt8<T>(x[qb][t][0], x[qb][t][1]));
+    }
+
+    // lane kt: the keys of tile kt that some row may see, this wave's half
+    // (dense masks reach this kernel with at most four tiles: lane 0 has their
+    // classes); a row whose own tile is not mixed has no word
+    uint32_t keys = ~0u;
+    if (MASKED && a.tile_keys) {
+        const uint32_t *p = (const uint32_t *)(a.tile_keys + (int64_t)plane * 2 * a.n_qt * a.n_kt) + (wave >> 1) +
+                            2 * min(lane, a.n_kt - 1);
+        uint32_t w[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) w[i] = p[2 * min(3 * qt + i, 2 * a.n_qt - 1) * a.n_kt];
+        const uint32_t sh = 8 * (uint32_t)(lane & 3);
+        const uint32_t c0 = (uint32_t)__builtin_amdgcn_readfirstlane(cls0) >> sh & 3u;
+        const uint32_t c1 = (uint32_t)__builtin_amdgcn_readfirstlane(cls1) >> sh & 3u;
+        keys = 0;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const uint32_t c = (3 * qt + i) / 2 == r0 ? c0 : c1;
+            keys |= c == 0 ? 0u : c == 1 ? ~0u : w[i];
+        }
     }
 
     // LDS operand addresses.  K operand (key block kb, dim step t): row
@@ -349,12 +382,12 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
     // (a look-ahead of 3 measured the same: C4 self 148.8-149.8 us against
     // 149.0)
     constexpr int kLook = 2, kRing = kLook + 1;
-    auto tile = [&](auto st_c, int kt, auto nst_c, int kn) __attribute__((always_inline)) {
+    auto tile = [&](auto st_c, int kt, auto nst_c, int kn, int cls) __attribute__((always_inline)) {
         constexpr int NST = decltype(nst_c)::value;
         const bool do_issue = kn < n_kt;   // uniform
         const uint32_t nl0 = lds0 + NST * kStageBytes + (uint32_t)(16 * wave) * 256u;
         const uint32_t nko = (uint32_t)(kn * kPfBN + 16 * wave) * k_row, nvo = (uint32_t)(kn * kPfBN + 16 * wave) * v_row;
-        const int cl = __builtin_amdgcn_readfirstlane(class_of(kt));
+        const int cl = cls & 3;
         const int key0 = kt * kPfBN;
         const bool general =
             __builtin_amdgcn_readfirstlane((int)(cl >= 2 || key0 + kPfBN > a.Skv || !lean_ok)) != 0;
@@ -503,21 +536,32 @@ __device__ __forceinline__ void fa_wide_body(const FaArgs a) {
     // of the tile, one barrier (every wave's copies have landed and every
     // wave is done with the other stage), compute, with the next live
     // tile's copies into the other stage spread over R1.
+    // V of keys that no row of the job sees, in stage ST (fa_prefill.h)
+    auto drop_dead = [&](int kt, int cls, int st) __attribute__((always_inline)) {
+        if (MODE == kWideNone || __builtin_expect(!(cls & kTileDeadKeys), 1)) return;
+        const uint32_t dead = SM ? dead_outside(sm_lo, sm_key_end, kt * kPfBN + 16 * wave)
+                                 : ~((uint32_t)__builtin_amdgcn_readlane(keys, kt) >> (16 * (wave & 1))) & 0xFFFFu;
+        zero_dead_v(dead, lds0 + (uint32_t)(st * kStageBytes + kTileBytes + 16 * wave * 256));
+    };
     std::integral_constant<int, 0> st0;
     std::integral_constant<int, 1> st1;
     int ofree = 1;   // the stage no tile still reads at the end
     while (kt < n_kt) {
         int kn = next_live(kt + 1);
+        int cls = __builtin_amdgcn_readfirstlane(class_of(kt));
         MXFA_WAIT_VMCNT(0);
+        drop_dead(kt, cls, 0);
         __builtin_amdgcn_s_barrier();
-        tile(st0, kt, st1, kn);
+        tile(st0, kt, st1, kn, cls);
         ofree = 1;
         kt = kn;
         if (kt >= n_kt) break;
         kn = next_live(kt + 1);
+        cls = __builtin_amdgcn_readfirstlane(class_of(kt));
         MXFA_WAIT_VMCNT(0);
+        drop_dead(kt, cls, 1);
         __builtin_amdgcn_s_barrier();
-        tile(st1, kt, st0, kn);
+        tile(st1, kt, st0, kn, cls);
         ofree = 0;
         kt = kn;
     }

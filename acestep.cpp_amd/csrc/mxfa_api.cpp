@@ -336,8 +336,9 @@ int check_norm_rope(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tenso
 
 struct Plan {
     bool prefill = false;
-    size_t cls_block = 0;   // prefill under a dense mask: tile classes, then (bits_off > 0) liveness words
+    size_t cls_block = 0;   // prefill under a dense mask: tile classes, then live keys and liveness words
     size_t bits_off = 0;
+    size_t keys_off = 0;    // > 0: the keys that 64-query rows see follow the classes
     size_t cls64_off = 0;   // > 0: the classes of 64-query tiles follow the first classes
     size_t part_off = 0;    // key-split prefill: partials after the classes
     bool narrow = false;    // prefill on the 16-query-per-wave kernel (fa_narrow.hip)
@@ -564,16 +565,24 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     // tile) follow the classes when the workspace can hold them; otherwise
     // the classifier labels such tiles 2
     const uint64_t bits_pf = mask ? (uint64_t)a.m_ne2 * a.m_ne3 * n_qt_pf * kPfBM * (uint64_t)n_kt * 8 : 0;
-    const uint64_t with_bits = ((cls_pf + 255) & ~255ull) + ((bits_pf + 255) & ~255ull);
+    // and between them, where they fit, the keys that some query of a 64-query
+    // row sees (8 bytes per row and key tile), by which V of masked slots is
+    // left out; odd mask rows are not taken without them (the decode kernel
+    // zeroes V of dead keys itself)
+    const uint64_t keys_pf = mask ? (uint64_t)a.m_ne2 * a.m_ne3 * 2 * n_qt_pf * (uint64_t)n_kt * 8 : 0;
+    const uint64_t keys_r = (keys_pf + 255) & ~255ull;
+    const bool keys_fit = mask && ((cls_pf + 255) & ~255ull) + keys_r + (q8 ? 512ull * (uint64_t)n_kv_rows : 0) <= ws_cap;
+    const uint64_t with_bits = ((cls_pf + 255) & ~255ull) + keys_r + ((bits_pf + 255) & ~255ull);
     // (Q8_0 calls keep reading mask values: their prefill instance has no
     // word path)
     const bool bits_fit = mask && !q8 && with_bits <= ws_cap;
     // the classes of 64-query tiles (fa_narrow.hip), where they fit as well
     const uint64_t cls64_pf = 2 * cls_pf;
-    const bool cls64_fit = mask && !q8 && ((cls_pf + cls64_pf + 255) & ~255ull) + ((bits_pf + 255) & ~255ull) <= ws_cap;
+    const bool cls64_fit =
+        mask && !q8 && ((cls_pf + cls64_pf + 255) & ~255ull) + keys_r + ((bits_pf + 255) & ~255ull) <= ws_cap;
     pl.prefill = (k->type == MXFA_TYPE_F16 || k->type == MXFA_TYPE_BF16 || q8) && a.Sq >= kPrefillMinSq &&
                  mask_vec_ok && offsets_32 && stage_ok && stage_fits && (!mask || n_kt <= kPfMaxKeyTiles) &&
-                 (!a.mask_unal || cls_pf <= ws_cap);
+                 (!a.mask_unal || keys_fit);
     if (pl.prefill) {
         a.n_qt = (a.Sq + kPfBM - 1) / kPfBM;
         a.n_kt = (int32_t)n_kt;
@@ -624,6 +633,10 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         if (cls64_fit) {
             pl.cls64_off = pl.ws_bytes;
             pl.ws_bytes += (size_t)cls64_pf;
+        }
+        if (keys_fit) {
+            pl.keys_off = (pl.ws_bytes + 255) & ~(size_t)255;
+            pl.ws_bytes = pl.keys_off + (size_t)keys_r;
         }
         if (bits_fit) {
             pl.bits_off = (pl.ws_bytes + 255) & ~(size_t)255;
@@ -1037,6 +1050,7 @@ int run(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const 
             uint8_t *cls64 = pl.cls64_off ? cls + pl.cls64_off : nullptr;
             a.tile_class64 = cls64;
             a.tile_bits = pl.bits_off ? (uint64_t *)(cls + pl.bits_off) : nullptr;
+            a.tile_keys = pl.keys_off ? (uint64_t *)(cls + pl.keys_off) : nullptr;
             if (classify) {
                 e = timed_launch("mask_classify", stream,
                                  [&] { return launch_mask_classify(a, pl.n_planes, cls, cls64, stream); });

@@ -97,6 +97,7 @@ struct FaArgs {
     // liveness word per query row (NULL: no words, no class 3)
     const uint8_t *tile_class;
     uint64_t *tile_bits;
+    uint64_t *tile_keys;                  // keys that some row of a 64-query half of a tile may see
     int32_t n_qt, n_kt;                   // tiles along Sq and Skv
     const uint8_t *tile_class64;          // the same classes per 64-query half of a tile (fa_narrow.hip)
     int32_t pf_parts, pf_tiles;           // fa_mfma.hip: key split, workgroups per job (0: none), live tiles per part

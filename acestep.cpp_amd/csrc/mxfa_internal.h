@@ -29,7 +29,12 @@ constexpr int kPfBN = 64;    // keys per K/V tile
 constexpr int kPfMaxKeyTiles = 512;   // class rows held in two registers per lane
 // With cls64, the class of each 64-query half of a tile goes to
 // cls64[(plane * 2 * n_qt + 2 * qt + half) * n_kt_pad + kt] as well, and the
-// words are written where the tile or either half is of class 3.
+// words are written where the tile or either half is of class 3.  With
+// a.tile_keys set, the keys that some row of a half may see (bit k: key k of
+// the tile) go to a.tile_keys[(plane * 2 * n_qt + 2 * qt + half) * n_kt + kt]
+// for tiles of class 2 and 3, and a class that leaves some key to no row at
+// all carries kTileDeadKeys.
+constexpr int kTileDeadKeys = 4;
 hipError_t launch_mask_classify(const FaArgs &a, int n_planes, uint8_t *classes, uint8_t *cls64,
                                 hipStream_t stream);
 
