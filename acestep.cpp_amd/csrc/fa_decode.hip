@@ -1077,13 +1077,15 @@ fa_decode_reg_kernel(const FaArgs a) {
         const u16x8 pbits = cvt8<TV>(p0, p1);
         lsum = sum8<TV>(pbits, lsum);
         const V8 pb = __builtin_bit_cast(V8, pbits);
-        // bf16: the lo parts of P for a second PV product (bf16_lo)
-        V8 pl = {};
-        if constexpr (TV == T_BF16) {
-            const u16x8 lbits = bf16_lo8(p0, p1, pbits);
-            lsum = sum8<TV>(lbits, lsum);
-            pl = __builtin_bit_cast(V8, lbits);
-        }
+        // the lo parts of P for a second PV product (p_lo8), in every type:
+        // with P rounded once the error grew with the keys that share a
+        // maximum, i.e. with the split (Q8_0, 32/8 heads, one token over 4096
+        // keys: 2.54e-4 of 64 bits in 64-key splits, 2.75e-4 in 128-key ones;
+        // with the pair 2.08e-4 for any split, V's own rounding.  4 sequences
+        // of 8192 keys: 22.9 -> 23.6 us).
+        const u16x8 lbits = p_lo8<TV>(p0, p1, pbits);
+        lsum = sum8<TV>(lbits, lsum);
+        const V8 pl = __builtin_bit_cast(V8, lbits);
 
         // V^T into this wave's LDS tile.  Chunk kc (4 keys) of row d is
         // stored at chunk slot kc ^ ((d >> 4) & 7).
@@ -1126,7 +1128,7 @@ fa_decode_reg_kernel(const FaArgs a) {
             u16x4 vhi = *(const u16x4 *)(row + 4 * ((g16 + 4) ^ dt));
             u16x8 av = {vlo[0], vlo[1], vlo[2], vlo[3], vhi[0], vhi[1], vhi[2], vhi[3]};
             o[dt] = MF::run(__builtin_bit_cast(V8, av), pb, o[dt]);
-            if constexpr (TV == T_BF16) o[dt] = MF::run(__builtin_bit_cast(V8, av), pl, o[dt]);
+            o[dt] = MF::run(__builtin_bit_cast(V8, av), pl, o[dt]);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();

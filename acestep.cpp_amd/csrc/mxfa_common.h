@@ -318,7 +318,7 @@ __device__ __forceinline__ u16x8 bf16_lo8(f32x4 lo4, f32x4 hi4, u16x8 hi) {
     for (int i = 0; i < 8; i++) r[i] = bf16_lo(i < 4 ? lo4[i] : hi4[i - 4], hi[i]);
     return r;
 }
-// the same for f16, which carries P to ~2^-22 so: the LDS decode kernel (its
+// the same for f16, which carries P to ~2^-22 so: the decode kernels (their
 // error then does not depend on how the keys are split) and the prefill
 // kernels under odd mask rows
 template <int T>
