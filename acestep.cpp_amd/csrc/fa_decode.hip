@@ -400,16 +400,20 @@ __device__ void merge_splits(const FaArgs &a, const Tile &t, int64_t pr0, int nr
         ml[j] = u32x2{0xFF800000u, 0u};   // m = -inf, l = 0
         if (r < nr && lane < ns) ml[j] = ld_dev2(a.part_ml + ((pr0 + r) * stride + lane) * 2);
     }
-    // O of row r, splits part + parts * (u0 + u): slots at or past ns read
-    // the last split's (weight zero)
+    // O of row r, splits part + parts * (u0 + u), agent scope (sc1): slots at
+    // or past ns are outside the buffer and read zero (another split's O under
+    // a zero weight would make its infinities NaN)
     u32x2 po[32];
     auto load_o = [&](int r, int u0) __attribute__((always_inline)) {
-        const float *p = a.part_o + (pr0 + r) * stride * kD + 2 * lane;
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc((void *)(a.part_o + (pr0 + r) * stride * kD), (short)0,
+                                                          ns * kD * 4, 0x00020000);
 #pragma unroll
         for (int v = 0; v < 32; v += 8) {
             if (part + parts * (u0 + v) >= ns) break;   // uniform
 #pragma unroll
-            for (int u = v; u < v + 8; u++) po[u] = ld_dev2(p + (int64_t)min(part + parts * (u0 + u), ns - 1) * kD);
+            for (int u = v; u < v + 8; u++)
+                po[u] = __builtin_bit_cast(
+                    u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, 8 * lane + (part + parts * (u0 + u)) * kD * 4, 0, 16));
         }
     };
     if (ra < nr) load_o(ra, 0);
@@ -519,21 +523,21 @@ __device__ void finish_tile(const FaArgs &a, const Tile &t, int ns, const f32x4 
     }
 
     // Several splits: partial out, then the tile's last workgroup merges.
-    // Every value that crosses workgroups is itself an agent-scope atomic
-    // access: the partials go out as agent-scope stores (global_store ... sc1,
+    // Every value that crosses workgroups is itself an agent-scope access: the
+    // partials go out as agent-scope stores (global_store ... sc1,
     // the encoding of a relaxed agent-scope atomic store on this
     // architecture, written through to the device coherence point), the
     // ticket is an agent-scope atomic add, and the merge reads the partials
-    // with agent-scope atomic loads (sc1, served from the coherence point,
-    // never from a stale L2 line).  A store counts in vmcnt until the
+    // with agent-scope loads ((m, l) atomic, O by buffer loads; sc1, served
+    // from the coherence point, never from a stale L2 line).  A store counts in vmcnt until the
     // coherence point has acknowledged it, so `s_waitcnt vmcnt(0)` in every
     // wave, then the barrier, put every partial at the coherence point before
     // thread 0 issues its ticket add; the workgroup that draws the last
     // ticket issues its loads after that add has returned.  The compiler
     // keeps this order: the waitcnt is an asm statement with a "memory"
-    // clobber, which no memory access may cross; the merge's loads are
-    // atomic (never speculated) and sit behind the ticket's value, which
-    // reaches every wave through LDS and a barrier.  The compiler's
+    // clobber, which no memory access may cross; the merge's loads (atomics
+    // and buffer intrinsics are never speculated) sit behind the ticket's
+    // value, which reaches every wave through LDS and a barrier.  The compiler's
     // release/acquire fences at agent scope would add a whole-L2 write-back
     // (buffer_wbl2) per wave and an L2 invalidate (buffer_inv) per ticket --
     // measured: C3 44.7 -> 140 us, C5 31 -> 57 us -- to cover ordinary
@@ -616,6 +620,7 @@ fa_decode_lds_kernel(const FaArgs a) {
     using MF = Mfma16<KT>;
     using V8 = typename MF::v8;
     using PV = Mfma16k16<KT>;
+    constexpr float kUp = pair_up<KT>();
     constexpr int kPer = 8 + (MM == kMaskVec ? 2 : 0);   // DMA instructions per stage
     static_assert(kD == 128, "kernel is written for D = 128");
 
@@ -785,8 +790,8 @@ fa_decode_lds_kernel(const FaArgs a) {
             bmax = fmaxf(bmax, xv);
         }
         bmax = max_half32(max_pair16(bmax));
-        if (__any(bmax > m2 + 8.0f)) {
-            const float mnew = fmaxf(m2, bmax);
+        if (__any(bmax > m2 + (8.0f + kUp))) {
+            const float mnew = fmaxf(m2, bmax - kUp);
             const float alpha = (mnew == -INFINITY) ? 1.0f : fast_exp2(m2 - mnew);
             m2 = mnew;
             lsum *= alpha;
@@ -797,15 +802,14 @@ fa_decode_lds_kernel(const FaArgs a) {
         f32x4 p;
 #pragma unroll
         for (int i = 0; i < 4; i++) p[i] = fast_exp2(xs[i] - m_use);   // exp2(-inf) = 0
-        const u16x8 pb8 = cvt8<KT>(p, f32x4{0.f, 0.f, 0.f, 0.f});
-        lsum = sum8<KT>(pb8, lsum);
-        const u16x4 pb = {pb8[0], pb8[1], pb8[2], pb8[3]};
-        // the lo parts of P for a second PV product (p_lo8).  In F16 too: P
+        // the hi and lo parts of P for two PV products (p_pair).  In F16 too: P
         // rounded once is less far off the fewer keys share a maximum, so
         // longer splits lost precision (28 layers over 1377 + 1290 keys:
         // 1.3e-4 of 64 bits in 64-key splits, 1.9e-4 in 192-key ones).
-        const u16x8 pl8 = p_lo8<KT>(p, f32x4{0.f, 0.f, 0.f, 0.f}, pb8);
-        lsum = sum8<KT>(pl8, lsum);
+        u16x8 pb8, pl8;
+        p_pair8<KT>(p, f32x4{0.f, 0.f, 0.f, 0.f}, pb8, pl8);
+        lsum = sum8<KT>(pl8, sum8<KT>(pb8, lsum));
+        const u16x4 pb = {pb8[0], pb8[1], pb8[2], pb8[3]};
         const u16x4 pl = {pl8[0], pl8[1], pl8[2], pl8[3]};
 
         // O^T[d][row] += V^T[d][keys 4*g16 + e] . P^T; V values of dead
@@ -902,6 +906,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 fa_decode_reg_kernel(const FaArgs a) {
     constexpr bool kQ8 = KT == T_Q8_0;
     constexpr int TV = kQ8 ? T_F16 : KT;        // format of the PV product
+    constexpr float kUp = pair_up<TV>();
     using MF = Mfma16<TV>;
     using V8 = typename MF::v8;
     using Blk = std::conditional_t<kQ8, BlkQ, BlkF>;
@@ -1059,8 +1064,8 @@ fa_decode_reg_kernel(const FaArgs a) {
                 bmax = fmaxf(bmax, xv);
             }
         bmax = max_half32(max_pair16(bmax));
-        if (__any(bmax > m2 + 8.0f)) {
-            const float mnew = fmaxf(m2, bmax);
+        if (__any(bmax > m2 + (8.0f + kUp))) {
+            const float mnew = fmaxf(m2, bmax - kUp);
             const float alpha = (mnew == -INFINITY) ? 1.0f : fast_exp2(m2 - mnew);
             m2 = mnew;
             lsum *= alpha;
@@ -1074,17 +1079,16 @@ fa_decode_reg_kernel(const FaArgs a) {
             p0[i] = fast_exp2(xs[0][i] - m_use);
             p1[i] = fast_exp2(xs[1][i] - m_use);
         }
-        const u16x8 pbits = cvt8<TV>(p0, p1);
-        lsum = sum8<TV>(pbits, lsum);
-        const V8 pb = __builtin_bit_cast(V8, pbits);
-        // the lo parts of P for a second PV product (p_lo8), in every type:
+        // the hi and lo parts of P for two PV products (p_pair), in every type:
         // with P rounded once the error grew with the keys that share a
         // maximum, i.e. with the split (Q8_0, 32/8 heads, one token over 4096
         // keys: 2.54e-4 of 64 bits in 64-key splits, 2.75e-4 in 128-key ones;
         // with the pair 2.08e-4 for any split, V's own rounding.  4 sequences
         // of 8192 keys: 22.9 -> 23.6 us).
-        const u16x8 lbits = p_lo8<TV>(p0, p1, pbits);
-        lsum = sum8<TV>(lbits, lsum);
+        u16x8 pbits, lbits;
+        p_pair8<TV>(p0, p1, pbits, lbits);
+        lsum = sum8<TV>(lbits, sum8<TV>(pbits, lsum));
+        const V8 pb = __builtin_bit_cast(V8, pbits);
         const V8 pl = __builtin_bit_cast(V8, lbits);
 
         // V^T into this wave's LDS tile.  Chunk kc (4 keys) of row d is

@@ -608,23 +608,27 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // probabilities of pair u (registers 2u, 2u+1) of a half, packed into
     // the P^T operand: k-slot 4u' + i <-> key 16kk + 8u' + 4h + i =
     // register 8kk + 4u' + i, i.e. operand kk holds registers 8kk..8kk+7.
-    // pl receives the lo parts (p_lo), which a second PV MFMA adds: bf16, and
+    // pl receives the lo parts (p_pair), which a second PV MFMA adds: bf16, and
     // f16 under odd mask rows.  Without them such calls were further from 64
     // bits than on the decode kernel, whose waves' own maxima round less (2 x
     // 1085 tokens under a window of 128, or over 238 keys: 1.9e-4 against
     // 1.7e-4; with them 2.4e-7, 28.9 -> 33.5 and 22.8 -> 25.4 us).
     constexpr bool kLo = T == T_BF16 || UNAL;
+    constexpr float kUp = kLo ? pair_up<T>() : 0.0f;
     auto pair = [&](const f32x16 &sc, int u, float g, float mneg, u16x8 (&pw)[2], u16x8 (&pl)[2])
                     __attribute__((always_inline)) {
         const float p0 = fast_exp2(fmaf(sc[2 * u], g, mneg));
         const float p1 = fast_exp2(fmaf(sc[2 * u + 1], g, mneg));
-        const uint16_t h0 = Mfma16<T>::from_f32(p0), h1 = Mfma16<T>::from_f32(p1);
-        pw[u >> 2][2 * (u & 3)] = h0;
-        pw[u >> 2][2 * (u & 3) + 1] = h1;
+        u16x2 h, l;
         if constexpr (kLo) {
-            pl[u >> 2][2 * (u & 3)] = p_lo<T>(p0, h0);
-            pl[u >> 2][2 * (u & 3) + 1] = p_lo<T>(p1, h1);
+            p_pair<T>(p0, p1, h, l);
+            pl[u >> 2][2 * (u & 3)] = l[0];
+            pl[u >> 2][2 * (u & 3) + 1] = l[1];
+        } else {
+            h = u16x2{Mfma16<T>::from_f32(p0), Mfma16<T>::from_f32(p1)};
         }
+        pw[u >> 2][2 * (u & 3)] = h[0];
+        pw[u >> 2][2 * (u & 3) + 1] = h[1];
     };
     // the denominator sums exactly the weights the PV product uses
     auto psum = [&](const u16x8 (&pw)[2], const u16x8 (&pl)[2]) __attribute__((always_inline)) -> float {
@@ -724,9 +728,9 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
 
         // ---- R3: tile max, reference update (rare rescale) ----
         const float bmax = max_pair32(fmaxf(mxa, half_max(sb))) * g;
-        const bool any_need = __builtin_amdgcn_ballot_w64(bmax > m2 + 8.0f) != 0;   // wave-uniform
+        const bool any_need = __builtin_amdgcn_ballot_w64(bmax > m2 + (8.0f + kUp)) != 0;   // wave-uniform
         if (any_need) {
-            const float mnew = fmaxf(m2, bmax);
+            const float mnew = fmaxf(m2, bmax - kUp);
             const float alpha = (m2 == -INFINITY) ? 1.0f : fast_exp2(m2 - mnew);
             m2 = mnew;
             lsum *= alpha;

@@ -47,6 +47,7 @@ template <int T, int MODE, bool CAP, int NST>
 __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
     constexpr bool SM = MODE == kNarrowSm, DENSE = MODE == kNarrowDense || MODE == kNarrowUnal;
     constexpr bool kLo = T == T_BF16 || MODE == kNarrowUnal;   // P as a hi/lo pair (fa_mfma.hip)
+    constexpr float kUp = kLo ? pair_up<T>() : 0.0f;
     constexpr int kPer = 8 + (DENSE ? 1 : 0);   // copies per stage
     using MF = Mfma16<T>;
     using V8 = typename MF::v8;
@@ -266,11 +267,19 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
     auto probs = [&](const f32x4 (&s)[2], int kb, float gs, float mneg, u16x8 &pw, u16x8 &pl)
                      __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float p = fast_exp2(fmaf(s[kb][i], gs, mneg));
-            const uint16_t h = MF::from_f32(p);
-            pw[4 * kb + i] = h;
-            if constexpr (kLo) pl[4 * kb + i] = p_lo<T>(p, h);
+        for (int i = 0; i < 4; i += 2) {
+            const float p0 = fast_exp2(fmaf(s[kb][i], gs, mneg));
+            const float p1 = fast_exp2(fmaf(s[kb][i + 1], gs, mneg));
+            u16x2 h, l;
+            if constexpr (kLo) {
+                p_pair<T>(p0, p1, h, l);
+                pl[4 * kb + i] = l[0];
+                pl[4 * kb + i + 1] = l[1];
+            } else {
+                h = u16x2{MF::from_f32(p0), MF::from_f32(p1)};
+            }
+            pw[4 * kb + i] = h[0];
+            pw[4 * kb + i + 1] = h[1];
         }
     };
     auto psum = [&](const u16x8 &pw, const u16x8 &pl) __attribute__((always_inline)) -> float {
@@ -361,9 +370,9 @@ __device__ __forceinline__ void fa_narrow_body(const FaArgs &a) {
 
         // ---- R3: tile max, reference update (rare) ----
         const float bmax = fmaxf(mxa, max8(sb)) * gs;
-        if (__builtin_amdgcn_ballot_w64(bmax > m2 + 8.0f) != 0) {   // wave-uniform
+        if (__builtin_amdgcn_ballot_w64(bmax > m2 + (8.0f + kUp)) != 0) {   // wave-uniform
             const float rmax = max_pair16(max_half32(bmax));         // over the query's four lanes
-            const float mnew = fmaxf(m2, rmax);
+            const float mnew = fmaxf(m2, rmax - kUp);
             const float alpha = (m2 == -INFINITY) ? 1.0f : fast_exp2(m2 - mnew);
             m2 = mnew;
             lsum *= alpha;

@@ -312,27 +312,44 @@ __device__ __forceinline__ u16x8 cvt8(f32x4 lo, f32x4 hi) {
 __device__ __forceinline__ uint16_t bf16_lo(float p, uint16_t h) {
     return __builtin_bit_cast(uint16_t, (__bf16)(p - __builtin_bit_cast(float, (uint32_t)h << 16)));
 }
-__device__ __forceinline__ u16x8 bf16_lo8(f32x4 lo4, f32x4 hi4, u16x8 hi) {
-    u16x8 r;
-#pragma unroll
-    for (int i = 0; i < 8; i++) r[i] = bf16_lo(i < 4 ? lo4[i] : hi4[i - 4], hi[i]);
-    return r;
-}
-// the same for f16, which carries P to ~2^-22 so: the decode kernels (their
-// error then does not depend on how the keys are split) and the prefill
-// kernels under odd mask rows
+// P of two keys as the PV product's operand pairs (raw bits): bf16 as above.
+// In f16, which carries P to ~2^-22 so (the decode kernels, whose error then
+// does not depend on how the keys are split, and the prefill kernels under odd
+// mask rows), hi is cut below p, not rounded: lo = RNE_f16(p - hi) >= p 2^-14
+// is then positive, and an infinity of V stays one in both products (inf * 0
+// or inf * -x would make it NaN).  So that lo is not rounded to 0 for small
+// weights, these kernels hold their maxima kPairUp low (pair_up): P is at most
+// 2^(8 + 7), and lo positive down to weights of 2^-18.  (hi rounded: one token
+// over 4096 keys 2.4e-7 of 64 bits; cut at p (1 - 2^-11) 3.0e-7, at 1 - 2^-14
+// 2.7e-7.)
+constexpr float kPairUp = 7.0f;
+template <int T> constexpr float pair_up() { return T == T_F16 ? kPairUp : 0.0f; }
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 template <int T>
-__device__ __forceinline__ uint16_t p_lo(float p, uint16_t h) {
-    if constexpr (T == T_BF16) return bf16_lo(p, h);
-    else return Mfma16<T_F16>::from_f32(p - h2f_bits(h));
+__device__ __forceinline__ void p_pair(float p0, float p1, u16x2 &hi, u16x2 &lo) {
+    if constexpr (T == T_BF16) {
+        hi = u16x2{Mfma16<T>::from_f32(p0), Mfma16<T>::from_f32(p1)};
+        lo = u16x2{bf16_lo(p0, hi[0]), bf16_lo(p1, hi[1])};
+    } else {
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        constexpr float kBelow = 1.0f - 0x1p-14f;
+        hi = __builtin_bit_cast(u16x2, __builtin_amdgcn_cvt_pkrtz(p0 * kBelow, p1 * kBelow));
+        const f32x2 r = {p0 - h2f_bits(hi[0]), p1 - h2f_bits(hi[1])};
+        lo = __builtin_bit_cast(u16x2, __builtin_convertvector(r, h2));
+    }
 }
 template <int T>
-__device__ __forceinline__ u16x8 p_lo8(f32x4 lo4, f32x4 hi4, u16x8 hi) {
-    if constexpr (T == T_BF16) return bf16_lo8(lo4, hi4, hi);
-    u16x8 r;
+__device__ __forceinline__ void p_pair8(f32x4 a, f32x4 b, u16x8 &hi, u16x8 &lo) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) r[i] = Mfma16<T_F16>::from_f32((i < 4 ? lo4[i] : hi4[i - 4]) - h2f_bits(hi[i]));
-    return r;
+    for (int i = 0; i < 4; i++) {
+        u16x2 h, l;
+        p_pair<T>(i < 2 ? a[2 * i] : b[2 * i - 4], i < 2 ? a[2 * i + 1] : b[2 * i - 3], h, l);
+        hi[2 * i] = h[0];
+        hi[2 * i + 1] = h[1];
+        lo[2 * i] = l[0];
+        lo[2 * i + 1] = l[1];
+    }
 }
 
 // Sum of 8 16-bit values of format T (the rounded probabilities that feed
