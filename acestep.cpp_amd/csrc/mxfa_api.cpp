@@ -130,6 +130,19 @@ constexpr int64_t kSplitTargets[3] = {512, 256, 128};
 constexpr int64_t kSplitMinKeys512 = 768, kSplitMinKeys512Rows = 512, kSplitMinKeys512Sm = 384, kSplitMinKeys512Q8 = 256;
 constexpr int64_t kSplitMinKeys256 = 256;
 constexpr int64_t kSplitFew = 8;   // this few splits may be short at 256 workgroups
+// From 257 to 511 streams no target leaves room for a second split, and some
+// CUs run two of them, others one.  Two splits each (2 to 4 workgroups per CU)
+// even that out.  LDS kernel: better once K and V are well past the chip's 32
+// MB of L2, whatever their division into streams (MB, one split against two,
+// us, F16 at 32 / 8 heads): 25 49 (58), 31 50 (49), 38 69 (73), 42 65 (58), 44
+// 54 (52), 50 89 (89), 63 94 (76), 84 124 (90), 100 169 (158), 115 130 (103).
+// Register kernel, which is bound by its own work: for long splits, and while
+// two fill less than half of a second round of 512 workgroups (Q8_0, 320
+// streams of 2048 keys 61.9 (62.5), 3072 87.1 (82.2), 4096 112 (102), 392
+// streams of 4096 113 (124); F16 under odd rows, 320 of 3071 137 (134), 360 of
+// 3071 127 (130), 320 of 4095 178 (171)).
+constexpr int64_t kTwoSplitsBytes = 40000000;
+constexpr int64_t kTwoSplitsKeysQ8 = 1536, kTwoSplitsKeys = 2048, kTwoSplitsMaxWgs = 768;
 constexpr int kSplitKeyQuantum = 128;  // register kernel: 4 waves x 32 keys
 constexpr int kSplitKeyQuantumLds = 64;  // LDS kernel: 4 waves x 16 keys
 constexpr int64_t kMaxDecodeSplits = 64;   // merge capacity of the decode kernel
@@ -341,6 +354,7 @@ struct Plan {
     size_t keys_off = 0;    // > 0: the keys that 64-query rows see follow the classes
     size_t cls64_off = 0;   // > 0: the classes of 64-query tiles follow the first classes
     size_t part_off = 0;    // key-split prefill: partials after the classes
+    bool two_splits = false;   // decode in two splits, which one would serve as well
     bool narrow = false;    // prefill on the 16-query-per-wave kernel (fa_narrow.hip)
     bool wide = false;   // prefill on the 48-query-per-wave kernel (fa_wide.hip)
     FaArgs args{};
@@ -731,6 +745,17 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
             n_splits = (a.Skv + chunk - 1) / chunk;
             if (long_enough(target, chunk, n_splits)) break;
         }
+        // between one and two workgroups per CU the targets leave one split
+        const int64_t half = round_q((a.Skv + 1) / 2);
+        const bool two = lds_kernel ? 512 * n_kv_rows > kTwoSplitsBytes
+                                    : half >= (q8 ? kTwoSplitsKeysQ8 : kTwoSplitsKeys) && 2 * base <= kTwoSplitsMaxWgs;
+        // (where the workspace holds the partials: one split needs none)
+        const size_t two_bytes = (size_t)a.B * a.Nkv * a.M * 2 * (kD + 2) * sizeof(float);
+        if (n_splits == 1 && base > kDecCus && base < 2 * kDecCus && half < a.Skv && two && two_bytes <= ws_cap) {
+            chunk = half;
+            n_splits = 2;
+            pl.two_splits = true;
+        }
     }
     a.n_splits = (int32_t)n_splits;
     a.chunk = (int32_t)chunk;
@@ -998,14 +1023,15 @@ int run(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const 
     } else {
         int rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
         // A workspace that cannot grow (under capture, or out of memory)
-        // leaves a key-split prefill to its unsplit form and a mask of odd
-        // rows to the decode kernel, which need less of it or none.
+        // leaves a key-split prefill to its unsplit form, a mask of odd rows
+        // to the decode kernel and two decode splits to one, which need less
+        // of it or none.
         if (rc != MXFA_OK && pl.args.pf_parts > 0) {
             pl = Plan{};
             make_plan(q, k, v, mask, params, dst, pl, sm, SIZE_MAX, false);
             rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
         }
-        if (rc != MXFA_OK && pl.prefill && pl.args.mask_unal) {
+        if (rc != MXFA_OK && (pl.prefill ? pl.args.mask_unal != 0 : pl.two_splits)) {
             pl = Plan{};
             make_plan(q, k, v, mask, params, dst, pl, sm, 0, false);
             rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);

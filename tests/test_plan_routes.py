@@ -1,0 +1,85 @@
+"""Which kernel a call takes and how its keys are split, seen through the host
+API compiled over a stub HIP runtime (tests/c/api_host.cpp): no GPU."""
+from __future__ import annotations
+
+import ctypes
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+torch = pytest.importorskip("torch")
+import mxfa  # noqa: E402
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+D = 128
+
+
+@pytest.fixture(scope="module")
+def api(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    so = str(tmp_path_factory.mktemp("api") / "api_host.so")
+    subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "--offload-arch=gfx950", "-std=c++17", "-O1", "-fPIC",
+                    "-I", os.path.join(REPO, "include"), "-I", os.path.join(REPO, "acestep.cpp_amd", "csrc"), "-shared",
+                    "-no-hip-rt", "-Wl,-Bsymbolic", os.path.join(REPO, "tests", "c", "api_host.cpp"), "-o", so], check=True)
+    lib = ctypes.CDLL(so)
+    lib.stub_log.restype = ctypes.c_char_p
+    lib.mxfa_last_error.restype = ctypes.c_char_p
+    return lib
+
+
+def _call(api, Sq, Skv, B=1, Nh=32, Nkv=8, kv=1, mask=None, entry="mxfa_flash_attn_ext", stream=1):
+    """Status and log of one call.  mask: None, or the entries per row (a dense
+    mask of that pitch)."""
+    row = 136 if kv == 8 else 2 * D
+    T = mxfa.DeviceView
+    q = T(0, (D, Sq, Nh, B), (4, 4 * D * Nh, 4 * D, 4 * D * Nh * Sq), 1 << 30).desc()
+    k = T(kv, (D, Skv, Nkv, B), (34 if kv == 8 else 2, row, row * Skv, row * Skv * Nkv), 1 << 31).desc()
+    v = T(kv, (D, Skv, Nkv, B), (34 if kv == 8 else 2, row, row * Skv, row * Skv * Nkv), 1 << 32).desc()
+    o = T(0, (D, Nh, Sq, B), (4, 4 * D, 4 * D * Nh, 4 * D * Nh * Sq), 1 << 33).desc()
+    m = mask and T(1, (mask, Sq, 1, B), (2, 2 * mask, 2 * mask * Sq, 2 * mask * Sq), 1 << 34).desc()
+    p = mxfa.make_params(D ** -0.5)
+    r = ctypes.byref
+    args = [r(q), r(k), r(v), r(m) if m else None, r(p)] + ([] if entry == "mxfa_reserve" else [r(o)])
+    rc = getattr(api, entry)(*args, ctypes.c_void_p(stream))
+    return rc, api.stub_log().decode()
+
+
+def _splits(log):
+    return int(re.search(r"decode splits=(\d+)", log).group(1))
+
+
+@pytest.fixture(autouse=True)
+def fresh(api):
+    api.stub_set(1 << 30, 0)
+    yield
+    api.stub_set(1 << 30, 0)
+    api.mxfa_release()
+    api.stub_log()
+
+
+# 257 .. 511 streams of 16 rows: two splits where they are the faster, one elsewhere
+@pytest.mark.parametrize("kv,mask,B,Sq,Skv,splits", [
+    (1, 0, 5, 32, 4096, 2), (1, 4096, 5, 32, 4096, 2), (30, 0, 5, 32, 2048, 2),
+    (1, 0, 5, 32, 1024, 1), (1, 0, 3, 60, 2048, 1), (1, 0, 7, 28, 2048, 2), (1, 0, 4, 40, 1024, 1),
+    (8, 0, 5, 32, 4096, 2), (8, 0, 5, 32, 2048, 1), (8, 0, 7, 28, 4096, 1),
+    (1, 4095, 5, 32, 4095, 2), (1, 2047, 5, 32, 2047, 1),
+    (1, 0, 4, 32, 4096, 2), (1, 0, 8, 32, 8192, 1),      # 256 and 512 streams: the targets' own
+])
+def test_two_splits_between_the_targets(api, kv, mask, B, Sq, Skv, splits):
+    rc, log = _call(api, Sq, Skv, B=B, kv=kv, mask=mask)
+    assert rc == 0 and _splits(log) == splits, log
+
+
+def test_two_splits_need_no_more_than_there_is(api):
+    # 504 streams' partials are past the fixed scratch, 320 streams' are not
+    assert _splits(_call(api, 36, 8192, B=7, entry="mxfa_flash_attn_ext_noalloc")[1]) == 1
+    assert _splits(_call(api, 32, 4096, B=5, entry="mxfa_flash_attn_ext_noalloc")[1]) == 2
+    # a stream whose workspace cannot grow under capture
+    api.stub_set(1 << 30, 1)
+    rc, log = _call(api, 32, 4096, B=5, stream=2)
+    assert rc == 0 and _splits(log) == 1
