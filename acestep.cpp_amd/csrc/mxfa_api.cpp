@@ -557,8 +557,22 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     // (Q8_0 calls under such masks stay on the decode kernel, whose integer
     // dots are closer to ggml's than the F16 staging below; the LM, which
     // owns the quantised cache, always pads its masks)
+    // Few streams of 16 rows, or few keys, stay on the decode kernel as well:
+    // the prefill's classifier is a launch of its own (~4 us) and its rows
+    // are dealt to few workgroups.  Decode against prefill, us, at 16 / 8
+    // heads (streams x keys): 72 x 65 8.4 (12.3), 128 x 127 9.0 (13.2), 208 x
+    // 201 12.7 (15.0), 64 x 2001 27.1 (35.0), 64 x 4001 38.4 (45.4), 104 x
+    // 1001 25.4 (30.3), 256 x 41 8.4 (12.1), 512 x 127 13.1 (13.6); past the
+    // lines 128 x 301 18.9 (16.8), 128 x 1701 38.0 (35.7), 336 x 333 21.6
+    // (17.5), 528 x 41 15.6 (12.6).  (Measured for one sequence at two and
+    // four query heads per KV head and for batches at two, the DiT's and the
+    // encoders', whose masks these are; other batches take the prefill.)
+    const int64_t streams = (int64_t)a.B * a.Nkv * ((a.M + 15) / 16);
+    const bool odd_small = a.mask_unal && (a.B == 1 || a.G == 2) &&
+                           (streams <= 64 || (streams <= 104 && a.Skv <= 2048) || (streams <= 208 && a.Skv <= 256) ||
+                            (streams <= 512 && a.Skv <= 128));
     const bool mask_vec_ok = !mask || (a.m_plane_bytes != 0 &&
-                                       (!a.mask_unal || (a.Skv >= 4 && k->type != MXFA_TYPE_Q8_0)));
+                                       (!a.mask_unal || (a.Skv >= 4 && k->type != MXFA_TYPE_Q8_0 && !odd_small)));
     const int64_t n_kt = (a.Skv + kPfBN - 1) / kPfBN;
     // the prefill kernel addresses one (batch, kv head)'s K and V rows with
     // 32-bit offsets from a buffer base: every row of every key tile must

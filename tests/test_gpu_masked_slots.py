@@ -40,7 +40,7 @@ def _poison(c, dead):
     (129, 333, (70, 331), "random", dict(Nh=64, Nkv=8)),
     (385, 512, (0, 461), "zeros", dict(Nh=64, Nkv=8, B=1)),
     # key split, and rows of more than 64 key tiles
-    (128, 1701, (3, 1630), "zeros", dict(B=1)),
+    (128, 1701, (3, 1630), "zeros", {}),
     (128, 1700, (0, 1699), "random", dict(B=1)),
     (64, 4500, (0, 4201), "zeros", dict(B=1, Nh=2, Nkv=1)),
     (65, 4501, (100, 4201), "zeros", dict(B=4, Nh=32, Nkv=1)),

@@ -29,10 +29,10 @@ BOUND = 2e-5   # bf16 pairs carry 2^-17 of each weight: 4.4e-6 rms
     (1, 7, 2048, None, 1, 32, 8),
     (30, 1, 4096, "random", 2, 32, 8),
     # prefills under odd rows
-    (1, 100, 301, "random", 1, 16, 8),
+    (1, 100, 301, "random", 2, 16, 4),
     (1, 300, 333, "causal", 2, 64, 8),
-    (1, 70, 1701, "random", 1, 8, 2),
-    (30, 100, 301, "random", 1, 16, 8),
+    (1, 70, 1701, "random", 2, 8, 2),
+    (30, 100, 301, "random", 2, 16, 4),
 ])
 def test_probabilities_keep_their_bits(mx, kv_type, Sq, Skv, mask, B, Nh, Nkv):  # noqa: F811
     import oracle

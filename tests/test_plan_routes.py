@@ -83,3 +83,21 @@ def test_two_splits_need_no_more_than_there_is(api):
     api.stub_set(1 << 30, 1)
     rc, log = _call(api, 32, 4096, B=5, stream=2)
     assert rc == 0 and _splits(log) == 1
+
+
+# odd mask rows: the prefill kernels from where they are the faster, either side of each line of the rule
+@pytest.mark.parametrize("B,Sq,Nh,Skv,decode", [
+    (1, 64, 16, 4001, True), (1, 65, 16, 2047, True), (1, 65, 16, 2049, False),
+    (1, 104, 16, 1001, True), (1, 105, 16, 1001, False), (1, 104, 16, 2049, False),
+    (1, 208, 16, 255, True), (1, 209, 16, 255, False), (1, 208, 16, 257, False),
+    (2, 256, 16, 127, True), (2, 257, 16, 127, False), (2, 256, 16, 129, False),
+    (1, 127, 32, 127, True), (1, 333, 32, 333, False), (4, 127, 16, 127, True), (4, 128, 32, 41, False),
+    (2, 125, 16, 41, True), (2, 1085, 16, 238, False), (1, 437, 16, 437, False),
+])
+@pytest.mark.parametrize("kv", [1, 30])
+def test_odd_mask_rows_route(api, kv, B, Sq, Nh, Skv, decode):
+    rc, log = _call(api, Sq, Skv, B=B, Nh=Nh, kv=kv, mask=Skv)
+    assert rc == 0 and ("decode" in log) == decode and ("classify" in log) != decode, log
+    # (rows of whole 4-value groups are not concerned)
+    pitch = (Skv + 3) & ~3
+    assert "decode" not in _call(api, Sq, Skv, B=B, Nh=Nh, kv=kv, mask=pitch)[1]
