@@ -809,6 +809,15 @@ int workspace_of(hipStream_t stream, Workspace **out) {
     return MXFA_OK;
 }
 
+// hipMalloc, whose failure is taken back from the runtime's last error: the
+// call may go on in a form that needs no memory, and its launches report that
+// error's state.
+hipError_t try_malloc(void **p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 // Tile classes of a dense mask within the stream's current graph.  Sets
 // *cls to NULL when no graph has begun on the stream (the call classifies
 // into its workspace as before); else to the mask's class bytes in the
@@ -843,7 +852,7 @@ int graph_classes(const mxfa_tensor *mask, int64_t Sq, int64_t Skv, size_t bytes
                         need);
         const size_t want = std::max<size_t>((size_t)64 << 10, 2 * need);
         void *p = nullptr;
-        const hipError_t e = hipMalloc(&p, want);
+        const hipError_t e = try_malloc(&p, want);
         if (e != hipSuccess) return fail(MXFA_ERR_NOMEM, "hipMalloc(%zu): %s", want, hipGetErrorString(e));
         if (w->arena) w->retired.push_back(w->arena);
         w->arena = (uint8_t *)p;
@@ -897,7 +906,7 @@ int ensure_workspace(size_t bytes, int64_t n_tickets, hipStream_t stream, void *
         size_t want = std::max(bytes + bytes / 4, 2 * ws.size);
         want = (want + 4095) & ~(size_t)4095;
         void *p = nullptr;
-        e = hipMalloc(&p, want);
+        e = try_malloc(&p, want);
         if (e != hipSuccess) return fail(MXFA_ERR_NOMEM, "hipMalloc(%zu): %s", want, hipGetErrorString(e));
         if (ws.ptr) ws.retired.push_back(ws.ptr);
         ws.ptr = p;
@@ -906,7 +915,7 @@ int ensure_workspace(size_t bytes, int64_t n_tickets, hipStream_t stream, void *
     if (ws.n_tickets < n_tickets) {
         const int64_t want = std::max<int64_t>(1024, n_tickets + n_tickets / 4);
         int *p = nullptr;
-        e = hipMalloc((void **)&p, (size_t)want * sizeof(int));
+        e = try_malloc((void **)&p, (size_t)want * sizeof(int));
         if (e != hipSuccess) return fail(MXFA_ERR_NOMEM, "hipMalloc(tickets): %s", hipGetErrorString(e));
         e = launch_fill_zero(p, want, stream);
         if (e != hipSuccess) {
@@ -1013,6 +1022,27 @@ int scratch_of_device(hipStream_t stream, Scratch *out) {
     return MXFA_OK;
 }
 
+// The stream's workspace for the plan `pl`.  One that cannot grow (under
+// capture, or out of memory) leaves a key-split prefill to its unsplit form, a
+// mask of odd rows to the decode kernel and two decode splits to one, which
+// need less of it or none: `pl` is then that form's plan.
+int fit_workspace(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const mxfa_tensor *mask,
+                  const mxfa_params *params, mxfa_tensor *dst, Plan &pl, const mxfa_mask_spec *sm, hipStream_t stream,
+                  void **ws, int **tickets) {
+    int rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, ws, tickets);
+    if (rc != MXFA_OK && pl.args.pf_parts > 0) {
+        pl = Plan{};
+        make_plan(q, k, v, mask, params, dst, pl, sm, SIZE_MAX, false);
+        rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, ws, tickets);
+    }
+    if (rc != MXFA_OK && (pl.prefill ? pl.args.mask_unal != 0 : pl.two_splits)) {
+        pl = Plan{};
+        make_plan(q, k, v, mask, params, dst, pl, sm, 0, false);
+        rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, ws, tickets);
+    }
+    return rc;
+}
+
 // Plans and launches one validated call (dense `mask` or structured `sm`).
 // `fixed`: use that scratch instead of the stream's grow-only workspace
 // (the allocation-free entry point); a call that needs more fails.
@@ -1035,21 +1065,7 @@ int run(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v, const 
         ws = fixed->ws;
         tickets = fixed->tickets;
     } else {
-        int rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
-        // A workspace that cannot grow (under capture, or out of memory)
-        // leaves a key-split prefill to its unsplit form, a mask of odd rows
-        // to the decode kernel and two decode splits to one, which need less
-        // of it or none.
-        if (rc != MXFA_OK && pl.args.pf_parts > 0) {
-            pl = Plan{};
-            make_plan(q, k, v, mask, params, dst, pl, sm, SIZE_MAX, false);
-            rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
-        }
-        if (rc != MXFA_OK && (pl.prefill ? pl.args.mask_unal != 0 : pl.two_splits)) {
-            pl = Plan{};
-            make_plan(q, k, v, mask, params, dst, pl, sm, 0, false);
-            rc = ensure_workspace(pl.ws_bytes, pl.n_tickets, stream, &ws, &tickets);
-        }
+        const int rc = fit_workspace(q, k, v, mask, params, dst, pl, sm, stream, &ws, &tickets);
         if (rc != MXFA_OK) return rc;
         if (!pl.prefill && (int64_t)pl.args.Nkv * pl.args.row_tiles > 65535)
             return fail(MXFA_ERR_UNSUPPORTED, "too many query rows per KV head for the decode kernel");
@@ -1190,7 +1206,7 @@ int mxfa_reserve(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *
     make_plan(q, k, v, mask, params, nullptr, pl);
     void *ws = nullptr;
     int *tickets = nullptr;
-    return ensure_workspace(pl.ws_bytes, pl.n_tickets, (hipStream_t)hip_stream, &ws, &tickets);
+    return fit_workspace(q, k, v, mask, params, nullptr, pl, nullptr, (hipStream_t)hip_stream, &ws, &tickets);
 }
 
 int mxfa_graph_begin(void *hip_stream) {

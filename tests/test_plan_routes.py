@@ -101,3 +101,32 @@ def test_odd_mask_rows_route(api, kv, B, Sq, Nh, Skv, decode):
     # (rows of whole 4-value groups are not concerned)
     pitch = (Skv + 3) & ~3
     assert "decode" not in _call(api, Sq, Skv, B=B, Nh=Nh, kv=kv, mask=pitch)[1]
+
+
+# (the first call's allocations: the workspace, then its tickets)
+@pytest.mark.parametrize("call,runs", [
+    (dict(Sq=128, Skv=1701, Nh=8, Nkv=2, B=2, mask=1701), {0: None, 1: "classify;prefill parts=0"}),
+    (dict(Sq=128, Skv=1700, Nh=8, Nkv=2, mask=1700), {0: None, 1: "classify;prefill parts=0"}),
+    (dict(Sq=128, Skv=1701, Nh=8, Nkv=2), {0: "wide", 1: "wide"}),
+    (dict(Sq=300, Skv=333, mask=333), {0: "decode splits=1"}),
+    (dict(Sq=32, Skv=4096, B=5), {0: "decode splits=1", 1: "decode splits=1"}),
+    (dict(Sq=1, Skv=4096), {0: None, 1: None}),
+])
+def test_no_memory_falls_back(api, call, runs):
+    for budget, run in runs.items():
+        for entry in ("mxfa_reserve", "mxfa_flash_attn_ext"):
+            api.mxfa_release()
+            api.stub_set(budget, 0)
+            rc, log = _call(api, entry=entry, stream=3, **call)
+            assert (rc == 0) == (run is not None), (budget, entry, api.mxfa_last_error())
+            assert entry == "mxfa_reserve" or run is None or log.startswith(run), (budget, log)
+
+
+def test_captured_calls_fall_back(api):
+    """No workspace yet and none to be had under capture: as without memory."""
+    api.stub_set(1 << 30, 1)
+    for entry in ("mxfa_reserve", "mxfa_flash_attn_ext"):
+        assert _call(api, 300, 333, mask=333, entry=entry, stream=4)[0] == 0
+        assert _call(api, 128, 1701, Nh=8, Nkv=2, entry=entry, stream=4)[0] == 0
+        assert _call(api, 300, 332, mask=332, entry=entry, stream=4)[0] != 0   # aligned rows: refused, as ever
+        assert _call(api, 1, 4096, entry=entry, stream=4)[0] != 0
