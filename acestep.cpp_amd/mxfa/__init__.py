@@ -226,10 +226,12 @@ class DeviceView:
     def desc(self) -> MxfaTensor:
         t = MxfaTensor()
         try:   # (one call for all ten fields: 0.5 us, field by field 1.6 us)
-            _TENSOR_FIELDS.pack_into(t, 0, self.type, *self.ne, *self.nb, self.ptr or 0)
-            return t
+            ne, nb = self.ne, self.nb
+            if len(ne) == 4 and len(nb) == 4:   # (5 + 3 values would fill the fields as well)
+                _TENSOR_FIELDS.pack_into(t, 0, self.type, *ne, *nb, self.ptr or 0)
+                return t
         except (struct.error, TypeError):
-            pass   # values that only int() takes, or out of a field's range
+            pass   # values that only int() takes, or out of a field's range, or of other lengths
         t.type = int(self.type)
         for i in range(4):
             t.ne[i] = int(self.ne[i])

@@ -44,3 +44,12 @@ def test_desc_refuses(view):
         _by_field(v)
     with pytest.raises(type(a.value)):
         v.desc()
+
+
+@pytest.mark.parametrize("ne,nb", [
+    ((128, 3, 2, 1, 2), (256, 768, 1536)),           # eight values in all, one on the wrong side
+    ((128, 3, 2), (1, 2, 256, 768, 1536)),
+])
+def test_desc_refuses_a_shifted_split(ne, nb):
+    with pytest.raises(IndexError):
+        mxfa.DeviceView(1, ne, nb, 4096).desc()
