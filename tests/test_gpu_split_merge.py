@@ -11,8 +11,10 @@ from test_gpu_parity import _rand_case, check, mx  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
+# (test_plan_routes.py holds the split counts: 66 and 130 are odd rows, 1 and 2
+# splits of the register kernel, the others 2 to 64 of the LDS kernel)
 
-@pytest.mark.parametrize("Skv", [66, 130, 2048, 2100, 4096, 6000])   # 2, 3, 32, 33, 64, 47 splits of the LDS kernel
+@pytest.mark.parametrize("Skv", [66, 68, 130, 132, 2048, 2100, 4096, 6000])
 @pytest.mark.parametrize("G,Sq", [(1, 1), (2, 1), (3, 1), (4, 1), (1, 7), (8, 2), (3, 6)])
 def test_merge_rows_and_splits(mx, G, Sq, Skv):  # noqa: F811
     c = _rand_case(900 + G + Sq + Skv, B=1, Sq=Sq, Nh=G, Nkv=1, Skv=Skv, mask="random")

@@ -75,6 +75,15 @@ def test_two_splits_between_the_targets(api, kv, mask, B, Sq, Skv, splits):
     assert rc == 0 and _splits(log) == splits, log
 
 
+# the merge tests' split counts at one and four streams
+@pytest.mark.parametrize("Skv,G,Sq,splits", [
+    (66, 1, 1, 1), (130, 1, 1, 2), (68, 1, 1, 2), (132, 1, 1, 3), (68, 8, 2, 2), (132, 3, 6, 3), (2048, 1, 1, 32),
+    (2100, 1, 1, 33), (4096, 1, 1, 64), (6000, 1, 1, 47), (4096, 8, 2, 64)])
+def test_merge_split_counts(api, Skv, G, Sq, splits):
+    rc, log = _call(api, Sq, Skv, Nh=G, Nkv=1, mask=Skv)
+    assert rc == 0 and _splits(log) == splits, log
+
+
 def test_two_splits_need_no_more_than_there_is(api):
     # 504 streams' partials are past the fixed scratch, 320 streams' are not
     assert _splits(_call(api, 36, 8192, B=7, entry="mxfa_flash_attn_ext_noalloc")[1]) == 1
