@@ -226,8 +226,8 @@ __device__ __forceinline__ void mfma_done(f32x16 &x) { asm volatile("s_nop 7\n\t
 // QQ8: Q quantised to Q8_0 on load, as ggml quantises Q for a Q8_0 K (the
 // K/V rows of a Q8_0 cache are staged in F16 by q8_stage.hip first).
 // UNAL: the dense mask's rows have no 8-byte alignment: values of mixed
-// tiles are read one by one (0 / -inf masks never get there: they come as
-// liveness words).
+// tiles are read one by one (0 / -inf masks come as liveness words and get
+// there only where a fixed scratch does not hold the words).
 // SPREAD: the next tile's copies go out one per QK MFMA of the current
 // tile (true), or all before the tile, with Q loaded as whole rows (false:
 // jobs of few key tiles, chosen in launch_fa_prefill).
@@ -612,7 +612,7 @@ __device__ __forceinline__ void fa_prefill_body(const FaArgs a) {
     // f16 under odd mask rows.  Without them such calls were further from 64
     // bits than on the decode kernel, whose waves' own maxima round less (2 x
     // 1085 tokens under a window of 128, or over 238 keys: 1.9e-4 against
-    // 1.7e-4; with them 2.4e-7, 28.9 -> 33.5 and 22.8 -> 25.4 us).
+    // 1.7e-4; with them 2.7e-7, 28.9 -> 33.5 and 22.8 -> 25.4 us).
     constexpr bool kLo = T == T_BF16 || UNAL;
     constexpr float kUp = kLo ? pair_up<T>() : 0.0f;
     auto pair = [&](const f32x16 &sc, int u, float g, float mneg, u16x8 (&pw)[2], u16x8 (&pl)[2])

@@ -18,8 +18,9 @@
 // ring of NST stages: four (132 KB, one workgroup per CU) where the grid has
 // at most one workgroup per CU, two (66 KB, two per CU) otherwise.  Kernel
 // times against the 128- and 192-query kernels: 437 tokens x 16 heads under a
-// window 12.4 against 16.3 us, without a mask 11.6 against 19.7 us; 333
-// tokens x 32 heads over 2133 keys 38.3 against 41.0 us.
+// window 12.4 against 16.3 us, without a mask 11.6 against 19.7 us.  (Few jobs
+// over many key tiles take fa_mfma.hip's key split: 333 tokens x 32 heads over
+// 2133 keys 30.8 us there, 38.3 here, 41.0 with neither.)
 //
 // Measured and dropped: two waves per query group, each with 32 queries and
 // half of a tile's keys, (m, l, O) merged at the end: half the LDS reads per

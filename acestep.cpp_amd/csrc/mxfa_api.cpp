@@ -546,9 +546,9 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
     // DiT's and the encoders' [S, S] masks for 3 of 4 lengths S.  Measured
     // per call against the scalar decode kernel, which streams all of K and
     // V for every 16 query rows: 2 x 1085 tokens at 16 / 8 heads under a
-    // window of 128, 33.7 against 123.7 us; over 238 encoder keys, 25.4
+    // window of 128, 34.3 against 123.7 us; over 238 encoder keys, 26.3
     // against 70.7 us; eight layers of 437 tokens, four of them under a
-    // window, 146.9 against 262.7 us.
+    // window, 98.0 against 262.7 us.
     if (mask) {
         const uint64_t plane = (uint64_t)(mask->ne[1] - 1) * mask->nb[1] + 2 * (uint64_t)mask->ne[0];
         a.m_plane_bytes = plane <= 0x7FFFFFFFull ? (uint32_t)plane : 0;
@@ -641,10 +641,11 @@ void make_plan(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_tensor *v,
         // nearly empty).  Measured, wide (128-query), 16 heads: 2 x 1250
         // tokens 41.6 (43.6) us, 2 x 1500 48.8 (52.0), 2 x 1700 74.7 (60.4),
         // 2 x 2000 88.7 (74.8), 2 x 2300 100.8 (114.4), 2 x 3000 144.5
-        // (157.2).  Masked calls keep it on every grid, which keeps a dense
-        // mask and its structured form bit-identical; that costs at most a
-        // few us (240 keys: 2 x 1085 24.0 (23.1), 2 x 2000 30.6 (26.3), 2 x
-        // 2300 30.8 (31.4), 2 x 3000 34.9 (37.6)).
+        // (157.2).  Masked calls over few key tiles keep it on every grid.  (A
+        // grid rule would serve a dense mask and its structured form alike, so
+        // their equality does not ask for this; over 240 keys it costs or
+        // gains: 2 x 1085 24.0 (23.1), 2 x 2000 30.6 (26.3), 2 x 2300 30.8
+        // (31.4), 2 x 3000 34.9 (37.6).)
         // (mask rows without 8-byte alignment: the 32-query kernel, which
         // reads the words of 0 / -inf tiles instead of their values)
         const int64_t jobs_w = (int64_t)((a.Sq + kPfWideBM - 1) / kPfWideBM) * a.Nh * a.B;

@@ -114,10 +114,13 @@ int mxfa_flash_attn_ext(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_t
  *   MXFA_MASK_LENGTHS  j < lengths[b % n_lengths]
  *   MXFA_MASK_CAUSAL   j <= pos0 + i
  *   MXFA_MASK_WINDOW   |pos0 + i - j| <= window
- * mxfa_flash_attn_ext_masked(q, k, v, spec, ...) computes exactly what
+ * mxfa_flash_attn_ext_masked(q, k, v, spec, ...) computes what
  * mxfa_flash_attn_ext(q, k, v, mask, ...) computes for the F16 mask
  * [Skv, Sq, 1, B] holding 0 at live keys and -inf elsewhere (flags == 0:
- * no mask).  Nothing is read from device memory for the mask: no mask
+ * no mask): with Sq >= 64 bit for bit where the mask's rows are 8-byte
+ * aligned and of a multiple of 4 entries, else within rounding (F16 calls
+ * under other rows carry P as two 16-bit parts; decode splits the keys by
+ * their live lengths).  Nothing is read from device memory for the mask: no mask
  * upload, no mask reads, no mask-classifier pass, and the split-KV decode
  * sizes its splits from the live lengths.  `lengths` is host memory read
  * during the call (n_lengths is 1 or B, at most 64; values >= 0); pos0 >= 0,
@@ -235,13 +238,19 @@ int mxfa_qk_norm_rope(const mxfa_tensor *q, const mxfa_tensor *k, const mxfa_ten
  * node arguments stay at fixed addresses and only their contents change
  * between replays (kv_rows, masks, positions).  Every mxfa entry point is
  * capture-safe -- kernels only, no memset, no host synchronisation, split
- * tickets reset by the kernels themselves -- except when the per-device
+ * tickets reset by the kernels themselves -- except when the stream's
  * workspace has to grow: that call fails with MXFA_ERR_UNSUPPORTED while
- * `hip_stream` is being captured.  mxfa_reserve() grows the workspace of
+ * `hip_stream` is being captured.  Three kinds of call run in a form that
+ * needs less workspace or none instead, slower and with other last bits: a
+ * prefill whose keys are split runs unsplit, a prefill under mask rows that
+ * are not 8-byte aligned or not of a multiple of 4 entries runs on the decode
+ * kernel, a decode of two splits for balance runs in one.  (The same forms
+ * serve when device memory is out.)  mxfa_reserve() grows the workspace of
  * `hip_stream` on the current device for the given FA call without
  * launching anything (beyond the one-time zero fill of a new ticket
- * buffer); so does any eager call of the same shapes on that stream.  A
- * graph keeps the workspace addresses of the stream it was captured on:
+ * buffer); so does any eager call of the same shapes on that stream.  (With
+ * mask == NULL it sizes a structured prefill of those shapes too; a
+ * structured decode is sized by an eager call.)  A graph keeps the workspace addresses of the stream it was captured on:
  * a later grow of that workspace retires the old buffers but keeps them
  * allocated until mxfa_release(), so the graph stays valid.  Replays must
  * not overlap in time with other mxfa calls on the capture stream.  A
